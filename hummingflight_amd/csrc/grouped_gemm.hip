@@ -1226,13 +1226,14 @@ __device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint
                 store_tile_row<EPI, CB>(a, acc[j], row0 + rl, col0, 0, SW ? row0 + rl : a.scatter_rows[row0 + rl]);
         }
     };
-    // Row-block counts in buckets (8 .. 12 or 10 exact, the near-uniform
-    // prefill's range; smaller ones rounded up to even): the extra blocks multiply rows
-    // that were not loaded and are never stored.
-    const int nb = nrb >= 8 ? nrb : (nrb + 1) & ~1;
+    // Row-block counts: exact from 4 on (a call's experts average any of them:
+    // at T = 3001, 94 rows, half have 6 blocks and 38 % have 7; 7 run as 8 cost
+    // 2.2 % of the layer), smaller ones rounded up to even: the extra block
+    // multiplies rows that were not loaded and are never stored.
+    const int nb = nrb >= 4 ? nrb : (nrb + 1) & ~1;
     static_for_desc<ROWS / 16>([&](auto n_c) {
         constexpr int NM = decltype(n_c)::value;
-        if constexpr (NM >= 8 || NM % 2 == 0) {
+        if constexpr (NM >= 4 || NM % 2 == 0) {
             if (nb == NM) kloop(std::integral_constant<int, NM>{});
         }
     });
