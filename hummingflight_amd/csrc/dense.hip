@@ -38,6 +38,19 @@ void dense_workspace_free() {
 // (288 / 384 / 768 items take two or three rounds of 256 workgroups).
 static int dense_gu_ksplit_auto(int T) { return T >= 64 && T <= kDenseTileRows ? 2 : 1; }
 
+// The one-group tiles (launch_fixed_gemm) for both GEMMs of a layer: its
+// matrices hold at least one N tile each and are worth it.
+static bool dense_fixed(int T, int I) {
+    const int d = g.cfg.d;
+    return I >= fixed_tile_cols(4, true) && d >= fixed_tile_cols(4, false) && fixed_worth(T, (size_t)I * d);
+}
+static FixedPlan dense_gu_plan(int T, int I, int max_splits) {
+    return plan_fixed_gemm(T, I, true, 4, g.cfg.d / kGemmTileK, max_splits, g.num_cus);
+}
+static FixedPlan dense_dn_plan(int T, int I, int max_splits) {
+    return plan_fixed_gemm(T, g.cfg.d, false, 4, I / kGemmTileK, max_splits, g.num_cus);
+}
+
 static int dense_workspace_reserve(int inter) {
     DenseWorkspace& w = g.dws;
     const int tokens = g.max_tokens > 1 && g.gws.xh ? g.max_tokens : 0;
@@ -46,12 +59,20 @@ static int dense_workspace_reserve(int inter) {
     hipError_t e = hipMalloc(&w.h1, sizeof(float) * (size_t)inter);
     if (e == hipSuccess && tokens) e = hipMalloc(&w.hh, 2 * (size_t)tokens * inter);
     if (e == hipSuccess && tokens) e = hipMalloc(&w.hl, 2 * (size_t)tokens * inter);
-    // Partials for up to 8 K splits of a short prompt (one M tile leaves the
-    // down projection 24 items), 2 of a long one.
-    const int part_rows = std::max(2 * tokens, std::min(8 * tokens, 4096));
+    // Partials: what the plans of the one-group tiles take, looked at every 16
+    // tokens (a call's plan keeps within them), and at least the 128-row
+    // kernel's 8 splits of a short prompt, 2 of a long one, and for gate/up two
+    // splits of a 256-row tile.
+    int part_rows = std::max(2 * tokens, std::min(8 * tokens, 4096));
+    int gu_part_rows = 2 * std::min(tokens, kDenseTileRows);
+    for (int t = 16; tokens && t < tokens + 16; t += 16) {
+        if (!dense_fixed(t, inter)) continue;
+        const int gu = dense_gu_plan(t, inter, kFixedMaxSplits).ksplit;
+        const int dn = dense_dn_plan(t, inter, kFixedMaxSplits).ksplit;
+        if (gu > 1) gu_part_rows = std::max(gu_part_rows, t * gu);
+        if (dn > 1) part_rows = std::max(part_rows, t * dn);
+    }
     if (e == hipSuccess && tokens) e = hipMalloc(&w.part, sizeof(float) * (size_t)part_rows * g.cfg.d);
-    int gu_part_rows = 0;
-    for (int t = 2; t <= tokens; ++t) gu_part_rows = std::max(gu_part_rows, t * dense_gu_ksplit_auto(t));
     if (e == hipSuccess && gu_part_rows > 0)
         e = hipMalloc(&w.gu_part, sizeof(float) * (size_t)gu_part_rows * 2 * inter);
     if (e != hipSuccess) {
@@ -117,6 +138,69 @@ static int dense_down_ksplit(int items, int stages, int T, int blocks) {
         if (e_ != hipSuccess) return fail_hip(e_, what); \
     } while (0)
 
+// Both GEMMs on the one-group tiles, x already split into gws.xh / xl.  Each
+// M tile multiplies the same weights, so what a call costs is how evenly its
+// tiles, N tiles and K splits fill the CUs (plan_fixed_gemm).  At 6144 x 12288
+// with FP32 activations, against the 128- and 256-row tiles before (us per
+// layer): T = 2 96 -> 93, 16 110 -> 99, 64 158 -> 117, 128 213 -> 156, 300 490
+// -> 310, 777 916 -> 580, 2048 1585 -> 1418, 4096 3040 -> 2720.
+static int dense_fixed_forward(LayerState& L, int T, float* out, hipStream_t s) {
+    const Cfg& c = g.cfg;
+    DenseWorkspace& w = g.dws;
+    GroupedWorkspace& gw = g.gws;
+    const int I = L.dense_inter, blocks = gemm_blocks(kPrefillTileRows);
+    Pending p;
+    auto args = [&](const FixedPlan& pl) {
+        GemmArgs a{};
+        a.tile_rows = pl.tile_rows;
+        a.m_tiles = pl.m_tiles;
+        a.n_tiles = pl.n_tiles;
+        a.ksplit = pl.ksplit;
+        a.rows_total = T;
+        return a;
+    };
+    // HFMOE_DENSE_GU_KSPLIT overrides gate/up's splits, within the partials.
+    const int gu_max = std::min(kFixedMaxSplits, std::max(1, w.gu_part_rows / T));
+    FixedPlan pl = dense_gu_plan(T, I, gu_max);
+    const int want = env_int("HFMOE_DENSE_GU_KSPLIT", pl.ksplit);
+    pl.ksplit = want >= 1 && want <= gu_max && want * 4 <= c.d / kGemmTileK ? want : 1;
+    GemmArgs gu = args(pl);
+    gu.K = c.d;
+    gu.N = I;
+    gu.a_hi = gw.xh;
+    gu.a_lo = gw.xl;
+    gu.a_lo_flag = gw.lo_flag;
+    gu.b_fixed0 = L.dev.sg;
+    gu.b_fixed1 = L.dev.su;
+    gu.b_ld = c.d;
+    gu.h_hi = w.hh;
+    gu.h_lo = w.hl;
+    gu.out_f32 = w.gu_part;
+    prof_begin(p, "dense_gateup_gemm", s);
+    HF_CHECK_LAUNCH(launch_fixed_gemm(pl.ksplit > 1 ? EPI_PARTIAL : EPI_SWIGLU, pl.ksplit > 1, 4, gu, blocks, s),
+                    "dense gate/up gemm");
+    if (pl.ksplit > 1) {
+        prof_begin(p, "dense_swiglu", s);
+        HF_CHECK_LAUNCH(launch_swiglu_splits(w.gu_part, pl.ksplit, T, I, w.hh, w.hl, s), "dense gate/up split sum");
+    }
+    pl = dense_dn_plan(T, I, std::min(kFixedMaxSplits, std::max(1, w.part_rows / T)));
+    GemmArgs dn = args(pl);
+    dn.K = I;
+    dn.N = c.d;
+    dn.a_hi = w.hh;
+    dn.a_lo = w.hl;
+    dn.b_fixed0 = L.dev.sd;
+    dn.b_ld = I;
+    dn.out_f32 = pl.ksplit > 1 ? w.part : out;
+    prof_begin(p, "dense_down_gemm", s);
+    HF_CHECK_LAUNCH(launch_fixed_gemm(EPI_PARTIAL, false, 4, dn, blocks, s), "dense down gemm");
+    if (pl.ksplit > 1) {
+        prof_begin(p, "dense_down_sum", s);
+        HF_CHECK_LAUNCH(launch_sum_splits(w.part, pl.ksplit, (size_t)T * c.d, out, s), "dense down split sum");
+    }
+    return HFMOE_OK;
+}
+
 int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t s) {
     const Cfg& c = g.cfg;
     DenseWorkspace& w = g.dws;
@@ -142,15 +226,13 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
         return HFMOE_OK;
     }
     GroupedWorkspace& gw = g.gws;
-    // Past one 128-row M tile, the 256-row tiles (HFMOE_DENSE_MIN_TOKENS): a
-    // second 128-row M tile streams all the weights again (at 6144 x 12288:
-    // T = 129 0.320 against 0.206 ms, 191 0.325 against 0.246), and the
-    // 256-row tiles were faster at every T from 256 to 1024; up to 128 tokens
-    // the 128-row kernel is (T = 128: 0.188 against 0.201 ms).
-    const int TR = T >= env_int("HFMOE_DENSE_MIN_TOKENS", kGemmTileRows + 1) ? kDenseTileRows : kGemmTileRows;
     const int I = L.dense_inter;
     prof_begin(p, "split_x", s);
     HF_CHECK_LAUNCH(launch_split_bf16(x, gw.xh, gw.xl, (size_t)T * c.d, gw.lo_flag, s), "split x");
+    if (dense_fixed(T, I)) return dense_fixed_forward(L, T, out, s);
+    // Layers too small for those tiles: past one 128-row M tile, the 256-row
+    // tiles (HFMOE_DENSE_MIN_TOKENS).
+    const int TR = T >= env_int("HFMOE_DENSE_MIN_TOKENS", kGemmTileRows + 1) ? kDenseTileRows : kGemmTileRows;
     GemmArgs gu{};
     gu.K = c.d;
     gu.N = I;

@@ -25,13 +25,14 @@
 //     straight into registers (L2-resident activations, row-gathered through
 //     a_rowmap), both 2-4 K stages ahead of the one multiplied;
 //   * 192 (M) x 256 or 384 (N) x 64 (K), 8 wavefronts (prefill GEMMs whose
-//     sizes do not fit the wide tiles, dense layers, LM head): both operands
-//     by DMA into LDS, wavefronts split 2 (row-block parity) x 4 (column
-//     groups) -- gemm_item_split below;
+//     sizes do not fit the wide tiles; 256 x 256 for one-group GEMMs too small
+//     for them): both operands by DMA into LDS, wavefronts split 2 (row-block
+//     parity) x 4 (column groups) -- gemm_item_split below;
 //   * 192 or 160 (M) x 512 (N) x 64 (K), 8 wavefronts of 64 weight rows each
 //     over all rows (prefill gate/up, 160-row tiles when x has a lo half;
-//     prefill down projection, 160-row tiles): weights through private
-//     per-wavefront LDS rings -- gemm_item_wide below.
+//     prefill down projection, 160-row tiles; dense layers and the LM head,
+//     up to 160 rows, or 128 x 640): weights through private per-wavefront LDS
+//     rings -- gemm_item_wide below.
 // Persistent workgroups walk per-XCD item lists, n fastest, so an M tile's
 // activations are reused within that XCD's L2 (item_range).
 //
@@ -555,8 +556,8 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void grouped_gemm_kernel(Gem
 //
 // ROWS = 192 for the MoE GEMMs: a routed expert's ~128 rows at T = 4096 fit
 // one tile with room to spare (an expert with more takes several M tiles and
-// re-reads its weights).  ROWS = 256 for one-group GEMMs (dense layers, LM
-// head), whose weights are re-read once per M tile.
+// re-reads its weights).  ROWS = 256 for one-group GEMMs too small for the
+// wide tiles, whose weights are re-read once per M tile.
 //
 // At T = 4096 the weight stream alone (this kernel's DMA pattern, no
 // multiplies) and the multiplies alone (no DMA) each take about 70 % of the
@@ -993,12 +994,36 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_split_kernel(GemmArgs a) 
 // kept for the second half, about 5 bytes per weight byte, as on the 384-row
 // split tiles).
 constexpr int kWideWaves = 8;
-constexpr int kWideWaveRows = kWideTileCols / kWideWaves;  // weight rows per wavefront
-constexpr int kWideHalfRows = kWideWaveRows / 2;           // weight rows per half-stage
+constexpr int kWideHalfRows = kWideTileCols / kWideWaves / 2;  // weight rows per half-stage
 constexpr int kWideWRing = 3;                              // half-stages per wavefront ring
 constexpr size_t kWideLds = 2 * (2 * (size_t)kPrefillTileRows * GBK +
                                  (size_t)kWideWaves * kWideWRing * kWideHalfRows * GBK);
 static_assert(kWideLds + 64 <= 160 * 1024, "wide LDS");
+
+// FP32 output rows of one K split (EPI_PARTIAL): row blocks j of tile row row0
+// on, a lane's columns col0 + 16 cb + 0 .. 3.  PAIR: the first half of the
+// column blocks are gate columns, the others the matching up columns, N
+// further in output rows of 2 N.
+template <int NM, int CB, bool PAIR>
+__device__ __forceinline__ void store_fixed(const GemmArgs& a, const f32x4_t (&acc)[NM][CB], int row0, int rows,
+                                            int col0, int ks, int fr) {
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        const int rl = 16 * j + fr;
+        if (rl >= rows) continue;
+        if constexpr (PAIR) {
+            f32x4_t* o =
+                reinterpret_cast<f32x4_t*>(a.out_f32 + ((size_t)ks * a.rows_total + row0 + rl) * 2 * a.N + col0);
+#pragma unroll
+            for (int cb = 0; cb < CB / 2; ++cb) {
+                o[4 * cb] = acc[j][cb];
+                o[4 * cb + a.N / 4] = acc[j][cb + CB / 2];
+            }
+        } else {
+            store_tile_row<EPI_PARTIAL, CB>(a, acc[j], row0 + rl, col0, ks, row0 + rl);
+        }
+    }
+}
 
 // Sub-step j = H * s + half multiplies A half `half` of K stage s.  The
 // first sub-step of a stage reads the wavefront's weight fragments of stage s
@@ -1013,37 +1038,44 @@ static_assert(kWideLds + 64 <= 160 * 1024, "wide LDS");
 // EPI_SWIGLU: the gate/up GEMM (x, one or two halves); EPI_SCATTER: the down
 // projection (h, two halves), each wavefront's 64 weight rows 64 consecutive
 // output columns (half-stage h: rows 32 h + [0, 32) of them).
-template <int EPI, int HALVES, class Setup>
-__device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint16_t* lds, int t, int wave,
-                                               Setup&& on_setup) {
-    static_assert(EPI == EPI_SWIGLU || (EPI == EPI_SCATTER && HALVES == 2), "wide tiles");
-    constexpr bool SW = EPI == EPI_SWIGLU;
-    constexpr int ROWS = HALVES == 1 ? kPrefillTileRows : kWideTileRows;
+// EPI_PARTIAL (grouped_gemm_fixed_kernel): K split ks of FP32 output rows, each
+// wavefront's 16 CB weight rows as in the down projection, or with PAIR as in
+// gate/up, the up columns stored N after the gate ones.
+// A tile that would reach past N is moved back to end there: the columns it
+// shares with the tile before it are computed twice, alike.
+template <int EPI, int HALVES, int ROWS, int CB, bool PAIR, class Setup>
+__device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int mt, int nt, int ks, uint16_t* lds, int t,
+                                               int wave, Setup&& on_setup) {
+    static_assert(EPI == EPI_SWIGLU || EPI == EPI_PARTIAL || (EPI == EPI_SCATTER && HALVES == 2), "wide tiles");
+    constexpr bool SW = EPI == EPI_SWIGLU || PAIR;
+    static_assert(!SW || CB == 4, "gate and up: two column blocks each");
+    constexpr int WROWS = 16 * CB;                  // weight rows per wavefront
+    constexpr int HROWS = WROWS / 2;                // weight rows per half-stage
+    constexpr int COLS = kWideWaves * WROWS / (SW ? 2 : 1);  // output columns per tile (SW: per matrix)
     constexpr int AST = ROWS * GBK;                 // elements per A sub-step slot
     constexpr int NAD = (ROWS / 8 + kWideWaves - 1) / kWideWaves;  // A DMAs (8 rows x 128 bytes) per wavefront
-    constexpr int NWH = kWideHalfRows / 8;          // weight DMAs per half-stage
+    constexpr int NWH = HROWS / 8;                  // weight DMAs per half-stage
     constexpr int NWS = wide_w_per_substep(HALVES);  // weight half-stages issued per sub-step
-    static_assert(NAD == 3 && NWH == 4, "the counts tests/split_pipeline checks the waits with");
-    constexpr int WHS = kWideHalfRows * GBK;        // elements per weight half-stage slot
-    constexpr int CB = kWideWaveRows / 16;          // column blocks per wavefront
+    static_assert(NAD <= 3 && NWH == CB, "the counts the waits are checked with (tests)");
+    constexpr int WHS = HROWS * GBK;                // elements per weight half-stage slot
     uint16_t* aring = lds;
     uint16_t* wring = lds + 2 * AST + wave * (kWideWRing * WHS);
     const int lane = t & 63;
     const int fr = lane & 15;
     const int fq = lane >> 4;
-    const int nk = a.K / GBK;
+    // K stages [kst, kst + nk) of the K split
+    const int nk_all = a.K / GBK;
+    const int kst = EPI == EPI_PARTIAL ? ks * nk_all / a.ksplit : 0;
+    const int nk = EPI == EPI_PARTIAL ? (ks + 1) * nk_all / a.ksplit - kst : nk_all;
     const int nj = nk * HALVES;
 
-    item = __builtin_amdgcn_readfirstlane(item);
-    const int nt = item % a.n_tiles;
-    const int mt = item / a.n_tiles;
     // (the tile table is read with vector loads: the kernel writes memory too)
     const int g = __builtin_amdgcn_readfirstlane(a.tile_group ? a.tile_group[mt] : 0);
-    const int row0 = __builtin_amdgcn_readfirstlane(a.tile_row0 ? a.tile_row0[mt] : mt * ROWS);
+    const int row0 = __builtin_amdgcn_readfirstlane(a.tile_row0 ? a.tile_row0[mt] : mt * a.tile_rows);
     const int row_end = __builtin_amdgcn_readfirstlane(a.group_end ? a.group_end[g] : a.rows_total);
-    const int rows = min(ROWS, row_end - row0);
+    const int rows = min(a.tile_rows, row_end - row0);
     const int nrb = (rows + 15) >> 4;
-    const int n0 = nt * (SW ? kWideTileCols / 2 : kWideTileCols);  // first output column of the tile
+    const int n0 = min(nt * COLS, a.N - COLS);  // first output column of the tile
     const uint16_t* b0 = a.b_tab ? a.b_tab[3 * g + a.b_which] : a.b_fixed0;  // gate (down) rows
     const uint16_t* b1 = !SW ? b0 : a.b_tab ? a.b_tab[3 * g + a.b_which + 1] : a.b_fixed1;  // up rows
 
@@ -1061,13 +1093,14 @@ __device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint
         const int r = 8 * (kWideWaves * i + wave) + dr;
         const int gr = row0 + min(r, rows - 1);
         const size_t src = (size_t)(a.a_rowmap ? a.a_rowmap[gr] : gr);
-        aoff[i] = (uint32_t)(2 * (src * a.K + dc * 8));
+        aoff[i] = (uint32_t)(2 * (src * a.K + kst * GBK + dc * 8));
     }
     // Weights: half-stage h of this wavefront is gate rows (h = 0) or the
-    // matching up rows (h = 1) n0 + 32 w + [0, 32), or down rows
-    // n0 + 64 w + 32 h + [0, 32); DMA i covers 8 of them.
-    const int wrow = n0 + (SW ? kWideHalfRows : kWideWaveRows) * wave + dr;
-    const uint32_t woff = (uint32_t)(2 * ((size_t)wrow * a.b_ld + dc * 8));
+    // matching up rows (h = 1) n0 + 32 w + [0, 32), or rows
+    // n0 + 64 w + 32 h + [0, 32) of the one matrix (CB = 4); DMA i covers 8
+    // of them.
+    const int wrow = n0 + (SW ? HROWS : WROWS) * wave + dr;
+    const uint32_t woff = (uint32_t)(2 * ((size_t)wrow * a.b_ld + kst * GBK + dc * 8));
     const __amdgpu_buffer_rsrc_t rw0 = raw_rsrc(uniform_ptr(b0));
     const __amdgpu_buffer_rsrc_t rw1 = raw_rsrc(uniform_ptr(b1));
     const __amdgpu_buffer_rsrc_t ra0 = raw_rsrc(a.a_hi);
@@ -1089,7 +1122,7 @@ __device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint
         if (q >= 2 * nk) return;
         const int s = q >> 1, h = q & 1;
         dma16(pick(h != 0, rw1, rw0), woff,
-              (uint32_t)s * (2 * GBK) + (uint32_t)(8 * i + (SW ? 0 : kWideHalfRows * h)) * wrow_bytes,
+              (uint32_t)s * (2 * GBK) + (uint32_t)(8 * i + (SW ? 0 : HROWS * h)) * wrow_bytes,
               wring + (q % kWideWRing) * WHS + i * 512);
     };
     auto issue_w = [&](int q) {
@@ -1134,7 +1167,11 @@ __device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint
             const uint16_t* w0 = wring + ((2 * s) % kWideWRing) * WHS;
             const uint16_t* w1 = wring + ((2 * s + 1) % kWideWRing) * WHS;
             auto wfrag = [&](int cb, int kh) {
-                return frag(cb < CB / 2 ? w0 : w1, 16 * (cb % (CB / 2)) + fr, kh * 4 + fq);
+                const int r = 16 * cb + fr;  // of the wavefront's WROWS
+                if constexpr (CB % 2 == 0)
+                    return frag(cb < CB / 2 ? w0 : w1, 16 * (cb % (CB / 2)) + fr, kh * 4 + fq);
+                else  // the middle block lies in both half-stages (HROWS is a multiple of 8)
+                    return frag(r < HROWS ? w0 : w1, r < HROWS ? r : r - HROWS, kh * 4 + fq);
             };
             auto dma = [&](auto&& f) {
                 asm volatile("" ::: "memory");
@@ -1218,12 +1255,16 @@ __device__ __forceinline__ void gemm_item_wide(const GemmArgs& a, int item, uint
         // Every load of the item has landed (the last stage waits for all).
         // SWIGLU: h columns n0 + 32 w + 16 cb + 4 fq + q from gate block cb
         // and up block cb + 2; SCATTER: y columns n0 + 64 w + 16 cb + 4 fq + q.
-        const int col0 = n0 + (SW ? kWideHalfRows : kWideWaveRows) * wave + 4 * fq;
+        const int col0 = n0 + (SW ? HROWS : WROWS) * wave + 4 * fq;
+        if constexpr (EPI == EPI_PARTIAL) {
+            if constexpr (NM > 0) store_fixed<NM, CB, PAIR>(a, acc, row0, rows, col0, ks, fr);
+        } else {
 #pragma unroll
-        for (int j = 0; j < NM; ++j) {
-            const int rl = 16 * j + fr;
-            if (rl < rows)
-                store_tile_row<EPI, CB>(a, acc[j], row0 + rl, col0, 0, SW ? row0 + rl : a.scatter_rows[row0 + rl]);
+            for (int j = 0; j < NM; ++j) {
+                const int rl = 16 * j + fr;
+                if (rl < rows)
+                    store_tile_row<EPI, CB>(a, acc[j], row0 + rl, col0, 0, SW ? row0 + rl : a.scatter_rows[row0 + rl]);
+            }
         }
     };
     // Row-block counts: exact from 4 on (a call's experts average any of them:
@@ -1260,7 +1301,9 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void grouped_gemm_wide_kernel(G
                 on_setup();
                 return;
             }
-            gemm_item_wide<EPI, HALVES>(b, item, wlds, t, wave, on_setup);
+            constexpr int ROWS = HALVES == 1 ? kPrefillTileRows : kWideTileRows;
+            item = __builtin_amdgcn_readfirstlane(item);
+            gemm_item_wide<EPI, HALVES, ROWS, 4, false>(b, item / b.n_tiles, item % b.n_tiles, 0, wlds, t, wave, on_setup);
             lds_barrier();
         };
         if (!b.item_ctr || !r.by_mtile) {
@@ -1281,6 +1324,49 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void grouped_gemm_wide_kernel(G
         items(b, std::integral_constant<int, 2>{});
     } else {
         items(a, std::integral_constant<int, 1>{});
+    }
+}
+
+// The wide tiles for one group whose rows all multiply the same weights (dense
+// layers, LM head): M tiles of a.tile_rows <= ROWS rows (T split evenly, so
+// that no tile is nearly empty), 128 CB weight rows (PAIR and SWIGLU: 256 gate
+// and 256 up rows), K splits of whole stages (they need not be even).  Items
+// are dealt statically, M tiles fastest, in one contiguous range per XCD: the
+// M tiles of a weight tile run side by side and stream it through that XCD's
+// L2 together.  LOM: the A lo half by the device flag (x) or always (h).
+// What bounds it: the multiplies from about 64 rows (777 rows, both halves:
+// 1.53 PFLOP/s of MFMA work in gate/up, 602 -> 350 us against 256-row tiles,
+// whose 4 M tiles were two rounds of 256 CUs), the weight stream below (16
+// rows: 5.9 TB/s; per layer 110 -> 99 us).
+constexpr size_t fixed_lds(int cb) {
+    return 2 * (2 * (size_t)fixed_tile_rows(cb) * GBK + (size_t)kWideWaves * kWideWRing * (8 * cb) * GBK);
+}
+template <int EPI, bool PAIR, int LOM, int CB>
+__global__ __launch_bounds__(64 * kWideWaves, 1) void grouped_gemm_fixed_kernel(GemmArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t flds[];  // fixed_lds(CB) bytes
+    constexpr int ROWS = fixed_tile_rows(CB);
+    static_assert(fixed_lds(CB) <= 160 * 1024, "LDS");
+    const int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const bool use_lo = LOM == kLoAlways || *a.a_lo_flag != 0u;
+    const int total = a.m_tiles * a.n_tiles * a.ksplit;
+    const int nxcd = gridDim.x >= 8 ? 8 : 1;
+    const int xcd = blockIdx.x % nxcd;
+    const int stride = (int)gridDim.x / nxcd + (xcd < (int)gridDim.x % nxcd ? 1 : 0);
+    const int chunk = (total + nxcd - 1) / nxcd;
+    const int end = min(total, (xcd + 1) * chunk);
+    for (int item = xcd * chunk + blockIdx.x / nxcd; item < end; item += stride) {
+        const int mt = item % a.m_tiles, rest = item / a.m_tiles;
+        const int ks = rest % a.ksplit, nt = rest / a.ksplit;
+        auto run = [&](auto halves_c) __attribute__((always_inline)) {
+            constexpr int HALVES = decltype(halves_c)::value;
+            gemm_item_wide<EPI, HALVES, ROWS, CB, PAIR>(a, mt, nt, ks, flds, t, wave, [] {});
+        };
+        if (LOM == kLoAlways || use_lo)
+            run(std::integral_constant<int, 2>{});
+        else if constexpr (LOM != kLoAlways)
+            run(std::integral_constant<int, 1>{});
+        lds_barrier();
     }
 }
 
@@ -1359,14 +1445,33 @@ __global__ void split_bf16_kernel(const float* __restrict__ x, uint16_t* __restr
 
 // out[i] = ((part[0][i] + part[1][i]) + part[2][i]) + ...: the K splits of a
 // PARTIAL GEMM ([ks][n] FP32) summed in split order, four values per thread
-// (n a multiple of 4, both arrays 16-byte aligned).
+// (n a multiple of 4, both arrays 16-byte aligned).  Eight splits' loads go
+// out before the first is added: with a short batch's few thousand values the
+// kernel is its chain of loads (24 splits of 2 x 2048: 7.4 us one by one).
+__device__ __forceinline__ f32x4_t split_sum(const f32x4_t* p, size_t stride, int ks) {
+    f32x4_t v = __builtin_nontemporal_load(p);
+    int k = 1;
+    for (; k + 8 <= ks; k += 8) {
+        f32x4_t w[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) w[u] = __builtin_nontemporal_load(p + (k + u) * stride);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += w[u];
+    }
+    f32x4_t w[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (k + u < ks) w[u] = __builtin_nontemporal_load(p + (k + u) * stride);
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (k + u < ks) v += w[u];
+    return v;
+}
+
 __global__ void sum_splits_kernel(const float* __restrict__ part, int ks, size_t n4, float* __restrict__ out) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
-        f32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(part) + i);
-        for (int k = 1; k < ks; ++k) v += __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(part) + k * n4 + i);
-        reinterpret_cast<f32x4_t*>(out)[i] = v;
-    }
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride)
+        reinterpret_cast<f32x4_t*>(out)[i] = split_sum(reinterpret_cast<const f32x4_t*>(part) + i, n4, ks);
 }
 
 hipError_t launch_sum_splits(const float* part, int ks, size_t n, float* out, hipStream_t s) {
@@ -1392,12 +1497,7 @@ __global__ void swiglu_splits_kernel(const float* __restrict__ part, int ks, int
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
         const size_t t = i / i4, c4 = i % i4;
         const size_t gi = t * 2 * i4 + c4;  // gate columns 4 c4.., up columns I + 4 c4..
-        f32x4_t gv = __builtin_nontemporal_load(p4 + gi);
-        f32x4_t uv = __builtin_nontemporal_load(p4 + gi + i4);
-        for (int k = 1; k < ks; ++k) {
-            gv += __builtin_nontemporal_load(p4 + k * split4 + gi);
-            uv += __builtin_nontemporal_load(p4 + k * split4 + gi + i4);
-        }
+        const f32x4_t gv = split_sum(p4 + gi, split4, ks), uv = split_sum(p4 + gi + i4, split4, ks);
         uint32_t hw[2], lw[2];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -1496,6 +1596,42 @@ static hipError_t launch_gemm_wide(const GemmArgs& a, int blocks, hipStream_t s)
         raised = true;
     }
     return launch(grouped_gemm_wide_kernel<EPI>, dim3(blocks), dim3(64 * kWideWaves), (uint32_t)kWideLds, s, a);
+}
+
+template <int EPI, bool PAIR, int LOM, int CB>
+static hipError_t launch_fixed_inst(const GemmArgs& a, int blocks, hipStream_t s) {
+    static bool raised = false;
+    if (!raised) {
+        hipError_t e =
+            hipFuncSetAttribute(reinterpret_cast<const void*>(grouped_gemm_fixed_kernel<EPI, PAIR, LOM, CB>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)fixed_lds(CB));
+        if (e != hipSuccess) return e;
+        raised = true;
+    }
+    return launch(grouped_gemm_fixed_kernel<EPI, PAIR, LOM, CB>, dim3(blocks), dim3(64 * kWideWaves),
+                  (uint32_t)fixed_lds(CB), s, a);
+}
+
+hipError_t launch_fixed_gemm(int epi, bool pair, int cb, const GemmArgs& a, int blocks, hipStream_t s) {
+    const bool sw = pair || epi == EPI_SWIGLU;
+    const size_t lim = (size_t)1 << 32;  // 32-bit byte offsets into each operand
+    if (a.b_tab || a.tile_group || a.tile_row0 || a.group_end || a.a_rowmap || !a.a_hi || !a.a_lo || a.m_tiles < 1 ||
+        a.ksplit < 1 || a.K % GBK || a.ksplit > a.K / GBK || a.tile_rows % 16 || a.tile_rows > fixed_tile_rows(cb) ||
+        (size_t)a.m_tiles * a.tile_rows < (size_t)a.rows_total ||
+        (size_t)(a.m_tiles - 1) * a.tile_rows >= (size_t)a.rows_total || a.N < fixed_tile_cols(cb, sw) ||
+        (size_t)a.n_tiles * fixed_tile_cols(cb, sw) < (size_t)a.N || (sw && (a.N % 4 || !a.b_fixed1)) ||
+        (epi == EPI_SWIGLU && a.ksplit != 1) || blocks < 1 || (size_t)a.N * (size_t)a.b_ld * 2 >= lim ||
+        (size_t)a.rows_total * (size_t)a.K * 2 >= lim)
+        return hipErrorInvalidValue;
+    const bool flag = a.a_lo_flag != nullptr;
+    if (epi == EPI_SWIGLU && cb == 4 && flag)
+        return launch_fixed_inst<EPI_SWIGLU, false, kLoByFlag, 4>(a, blocks, s);
+    if (epi != EPI_PARTIAL) return hipErrorInvalidValue;
+    if (pair && cb == 4 && flag) return launch_fixed_inst<EPI_PARTIAL, true, kLoByFlag, 4>(a, blocks, s);
+    if (!pair && cb == 5 && flag) return launch_fixed_inst<EPI_PARTIAL, false, kLoByFlag, 5>(a, blocks, s);
+    if (!pair && cb == 4 && flag) return launch_fixed_inst<EPI_PARTIAL, false, kLoByFlag, 4>(a, blocks, s);
+    if (!pair && cb == 4 && !flag) return launch_fixed_inst<EPI_PARTIAL, false, kLoAlways, 4>(a, blocks, s);
+    return hipErrorInvalidValue;
 }
 
 template <int EPI, int LOM>

@@ -78,6 +78,9 @@ struct LmHead {
     int vocab = 0;
     void* part = nullptr;            // per-block winners of the T = 1 GEMV
     int part_n = 0;                  // their number: the most workgroups that GEMV takes
+    float* split = nullptr;          // K-split partials of the multi-token GEMM, or null
+    size_t split_floats = 0;
+    float* split_own = nullptr;      // the allocation behind them, if they have one
 };
 
 // Buffers of the dense-MLP layers (sized for the largest registered inter).

@@ -1,13 +1,13 @@
 // hf_grouped.h -- multi-token MoE: dispatch and the BF16 MFMA grouped GEMM.
 #pragma once
 
+#include "fixed_plan.h"
 #include "hf_common.h"
 
 namespace hf {
 
-constexpr int kGemmTileRows = 128;  // M rows per grouped-GEMM tile (kPrefillTileRows at prefill sizes)
 // Prefill tiles: 192 rows (a routed expert's rows at T = 4096 in one tile);
-// one-group GEMMs (dense layers, LM head) with T >= 192: 256 rows.
+// one-group GEMMs too small for launch_fixed_gemm's tiles: 256 rows.
 constexpr int kPrefillTileRows = 192, kDenseTileRows = 256;
 constexpr int kGemmTileK = 64;      // K per pipeline stage (K % (64 * ksplit) == 0)
 
@@ -101,6 +101,11 @@ struct GemmArgs {
 
 // Groups whose b_tab entry (3g + b_which) is null are skipped.
 hipError_t launch_grouped_gemm(int epi, const GemmArgs& a, int blocks, hipStream_t s);
+// One group, fixed B (grouped_gemm_fixed_kernel): M tiles of a.tile_rows rows, N
+// tiles of fixed_tile_cols(cb, pair) columns, a.ksplit K splits (PARTIAL).
+// pair (PARTIAL): b_fixed0 / b_fixed1 are gate and up, N rows each, and the
+// output rows [2 N] hold the gate columns, then the up ones.
+hipError_t launch_fixed_gemm(int epi, bool pair, int cb, const GemmArgs& a, int blocks, hipStream_t s);
 // p[0, n) = 0 by a kernel (graph-capture safe, unlike a memset node).
 hipError_t launch_clear_u32(unsigned* p, int n, hipStream_t s);
 // out[i] = sum over k < ks of part[k * n + i], in k order (n a multiple of 4).

@@ -13,8 +13,8 @@
 //   once and kept out of the caches' way); lane 0 writes the logit and
 //   keeps the wavefront's running winner, the block merges its four, and one
 //   small launch merges the blocks' winners (lowest row on equal values).
-// T > 1: the grouped GEMM (one group, fixed B = lm_head) writes the logits,
-//   then one block per token finds its argmax.
+// T > 1: a GEMM (one group, fixed B = lm_head) writes the logits, then one
+//   block per token finds its argmax.
 #include "hf_api_internal.h"
 #include "hf_grouped.h"
 
@@ -209,6 +209,7 @@ static int lm_call_grid() { return std::max(1, std::min(lm_grid(), g.lm.part_n))
 
 void lm_head_release() {
     if (g.lm.part) hipFree(g.lm.part);
+    if (g.lm.split_own) hipFree(g.lm.split_own);
     g.lm = LmHead{};
 }
 
@@ -218,6 +219,34 @@ void lm_head_release() {
         prof_end(p, s);                                  \
         if (e_ != hipSuccess) return fail_hip(e_, what); \
     } while (0)
+
+// The one-group tiles for T tokens, of 4 or 5 column blocks (cb), whichever the
+// estimate says (at the GLM vocabulary 242 tiles of 640 rows are one round of
+// 256 CUs, 303 of 512 two); cb = 0: the 128-row kernel, for a table or batch
+// too small for them.  Up to 16 tokens its first wavefront alone, with one
+// 16-row block, keeps up with the table's stream, on two workgroups per CU
+// (154880 x 6144: T = 2 310 against 326 us, 8 326 against 331, 16 339 against
+// 335-350, 24 377 against 335, 64 490 against 361, 128 690 against 430; T =
+// 300 1673 on 256-row tiles against 1114).
+constexpr int kLmFixedTokens = 17;
+constexpr size_t kLmSplitFloats = (size_t)64 << 20;  // K-split partials: as many are plenty
+static FixedPlan lm_plan(int T, int d, int vocab, size_t split_floats, int& cb) {
+    FixedPlan best;
+    cb = 0;
+    if (T < kLmFixedTokens || !fixed_worth(T, (size_t)vocab * d)) return best;
+    for (int c = 4; c <= 5; ++c) {
+        if (vocab < fixed_tile_cols(c, false) || (c == 5 && T > fixed_tile_rows(5))) continue;
+        // (the split sum adds four logits at a time)
+        const size_t one = (size_t)T * vocab;
+        const int splits = one % 4 ? 1 : (int)std::max((size_t)1, std::min((size_t)kFixedMaxSplits, split_floats / one));
+        const FixedPlan pl = plan_fixed_gemm(T, vocab, false, c, d / kGemmTileK, splits, g.num_cus);
+        if (!cb || pl.us < best.us) {
+            best = pl;
+            cb = c;
+        }
+    }
+    return best;
+}
 
 static int lm_head_forward(const float* h, int T, float* logits, int* token, hipStream_t s) {
     const Cfg& c = g.cfg;
@@ -246,18 +275,9 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     GroupedWorkspace& gw = g.gws;
     prof_begin(p, "split_x", s);
     HF_CHECK_LAUNCH(launch_split_bf16(xn, gw.xh, gw.xl, (size_t)T * c.d, gw.lo_flag, s), "split x");
-    // Past one 128-row M tile, the 256-row tiles (HFMOE_LM_MIN_TOKENS): a
-    // second 128-row M tile streams the whole table again (GLM vocab:
-    // T = 129-191 1.53-1.56 ms against 0.89-1.03 on one 256-row tile; up to
-    // 128 tokens the two are even, 0.77-0.88 ms).
-    const int TR = T >= env_int("HFMOE_LM_MIN_TOKENS", kGemmTileRows + 1) ? kDenseTileRows : kGemmTileRows;
     GemmArgs a{};
     a.K = c.d;
     a.N = L.vocab;
-    a.tile_rows = TR;
-    a.tile_cols = gemm_tile_cols(TR, EPI_PARTIAL);
-    a.n_tiles = gemm_n_tiles(EPI_PARTIAL, L.vocab, a.tile_cols);
-    a.m_tiles = (T + TR - 1) / TR;
     a.rows_total = T;
     a.a_hi = gw.xh;
     a.a_lo = gw.xl;
@@ -266,8 +286,31 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     a.b_ld = c.d;
     a.out_f32 = logits;
     a.ksplit = 1;
-    prof_begin(p, "lm_head_gemm", s);
-    HF_CHECK_LAUNCH(launch_grouped_gemm(EPI_PARTIAL, a, gemm_blocks(TR), s), "lm head gemm");
+    int cb = 0;
+    const FixedPlan pl = lm_plan(T, c.d, L.vocab, L.split_floats, cb);
+    if (cb) {
+        a.tile_rows = pl.tile_rows;
+        a.m_tiles = pl.m_tiles;
+        a.n_tiles = pl.n_tiles;
+        a.ksplit = pl.ksplit;
+        if (pl.ksplit > 1) a.out_f32 = L.split;
+        prof_begin(p, "lm_head_gemm", s);
+        HF_CHECK_LAUNCH(launch_fixed_gemm(EPI_PARTIAL, false, cb, a, gemm_blocks(kPrefillTileRows), s), "lm head gemm");
+        if (pl.ksplit > 1) {
+            prof_begin(p, "lm_head_sum", s);
+            HF_CHECK_LAUNCH(launch_sum_splits(L.split, pl.ksplit, (size_t)T * L.vocab, logits, s), "lm head split sum");
+        }
+    } else {
+        // Past one 128-row M tile (a table shorter than one 512-row tile), the
+        // 256-row tiles (HFMOE_LM_MIN_TOKENS).
+        const int TR = T >= env_int("HFMOE_LM_MIN_TOKENS", kGemmTileRows + 1) ? kDenseTileRows : kGemmTileRows;
+        a.tile_rows = TR;
+        a.tile_cols = gemm_tile_cols(TR, EPI_PARTIAL);
+        a.n_tiles = gemm_n_tiles(EPI_PARTIAL, L.vocab, a.tile_cols);
+        a.m_tiles = (T + TR - 1) / TR;
+        prof_begin(p, "lm_head_gemm", s);
+        HF_CHECK_LAUNCH(launch_grouped_gemm(EPI_PARTIAL, a, gemm_blocks(TR), s), "lm head gemm");
+    }
     if (token) {
         prof_begin(p, "lm_argmax", s);
         HF_CHECK_LAUNCH(launch_row_argmax(logits, T, L.vocab, token, s), "argmax");
@@ -292,6 +335,29 @@ int hfmoe_register_lm_head(const uint16_t* lm_head_dev, const uint16_t* final_no
     const int part_n = std::max(1, lm_grid());
     hipError_t e = hipMalloc(&g.lm.part, sizeof(ArgMax) * (size_t)part_n);
     if (e != hipSuccess) return fail_hip(e, "lm head workspace");
+    // K-split partials of the multi-token GEMM: the MoE path's y rows where
+    // they are plenty, else a buffer for what the plans take.
+    const size_t y_floats = g.gws.xh ? (size_t)g.max_tokens * (g.cfg.k + g.cfg.n_shared) * g.cfg.d : 0;
+    if (y_floats >= kLmSplitFloats) {
+        g.lm.split = g.gws.y;
+        g.lm.split_floats = y_floats;
+    } else if (g.gws.xh) {
+        size_t floats = 0;
+        for (int t = 32; t <= std::min((g.max_tokens + 15) / 16 * 16, 512); t += 16) {
+            int cb = 0;
+            const FixedPlan pl = lm_plan(t, g.cfg.d, vocab, kLmSplitFloats, cb);
+            if (pl.ksplit > 1) floats = std::max(floats, (size_t)pl.ksplit * t * vocab);
+        }
+        if (floats) {
+            e = hipMalloc(&g.lm.split_own, sizeof(float) * floats);
+            if (e != hipSuccess) {
+                lm_head_release();
+                return fail_hip(e, "lm head workspace");
+            }
+            g.lm.split = g.lm.split_own;
+            g.lm.split_floats = floats;
+        }
+    }
     g.lm.part_n = part_n;
     g.lm.w = lm_head_dev;
     g.lm.norm = final_norm_dev;
