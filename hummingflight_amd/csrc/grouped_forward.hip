@@ -43,21 +43,37 @@ int gemm_blocks(int tile_rows) {
     return env_int("HFMOE_GEMM_BLOCKS", tile_rows == kGemmTileRows ? g.num_cus * 2 : g.num_cus);
 }
 
-// Prefill tiles (192 rows; the wide tiles' own list 160) once experts
-// average 4+ rows (HFMOE_PREFILL_MIN_ROWS): an expert's rows then mostly fit
-// one tile, its weights stream through the memory system once, and each
-// activation row is requested once per 512 weight rows (the wide tiles; 256
-// or 384 on the split tiles).  Measured at full shape (256 experts top-8,
-// near-uniform routing): from 3 to 6 rows per expert the 128-row kernel
-// (whose wavefronts skip the row blocks a group does not fill) and the
-// prefill tiles are even; from 7 on the prefill tiles win by more the more
-// rows an expert has (T = 224: +4.5 %, 512: +15 %, 1024: +30 %, 2048: +39 %,
-// 2560: +34 % tokens/s).  Batched decode with skewed popularity (T = 64,
-// Zipf) stays on the 128-row kernel.
+// Prefill tiles (192 rows; the wide tiles' own list 160) or the 128-row kernel
+// for a batch: by the rows an expert averages and by how many of the prefill
+// tiles' large items (a whole expert's rows against 512 weight rows, one
+// workgroup per CU) there are to fill the CUs with.
+//   * Many (4 rounds of the CUs or more; the GLM-5.2 layer has 2056 items):
+//     from 4 rows on.  An expert's rows mostly fit one tile, its weights stream
+//     through the memory system once, and each activation row is requested
+//     once per 512 weight rows (the wide tiles; 256 or 384 on the split
+//     tiles).  Full shape (256 experts top-8, near-uniform routing): from 3 to
+//     6 rows per expert the 128-row kernel (whose wavefronts skip the row
+//     blocks a group does not fill) and the prefill tiles are even; from 7 on
+//     the prefill tiles win by more the more rows an expert has (T = 224:
+//     +4.5 %, 512: +15 %, 1024: +30 %, 2048: +39 %, 2560: +34 % tokens/s).
+//   * Fewer, but a round of them: from 96 rows on, where the multiplies count.
+//     64 experts of 2048 x 1024 have 264 items, one round and a tail as long,
+//     against 1072 of the 128-row kernel's: T = 32 264 against 196 us, 100 282
+//     / 229, 300 340 / 271, 500 (62 rows) 333 / 304, 1000 (125 rows) 413 / 465.
+//   * Less than a round: never (32 experts of 512 x 256, T = 64 91 against 49
+//     us, T = 1000 131 / 76).
+// HFMOE_PREFILL_MIN_ROWS sets the rows alone, whatever the items.  Batched
+// decode with skewed popularity (T = 64, Zipf) stays on the 128-row kernel.
 static int expert_tile_rows(int T) {
     const Cfg& c = g.cfg;
-    const int min_rows = env_int("HFMOE_PREFILL_MIN_ROWS", 4);
-    return (size_t)T * c.k >= (size_t)min_rows * c.E ? kPrefillTileRows : kGemmTileRows;
+    const size_t pairs = (size_t)T * c.k;
+    const int min_rows = env_int("HFMOE_PREFILL_MIN_ROWS", 0);
+    if (min_rows > 0) return pairs >= (size_t)min_rows * c.E ? kPrefillTileRows : kGemmTileRows;
+    const size_t per_expert = (pairs / c.E + kPrefillTileRows - 1) / kPrefillTileRows;
+    const size_t shared = c.n_shared > 0 ? ((size_t)T + kPrefillTileRows - 1) / kPrefillTileRows : 0;
+    const size_t items = ((size_t)c.E * per_expert + shared) * ((c.I + kWideTileCols / 2 - 1) / (kWideTileCols / 2));
+    const size_t rows = items >= 4 * (size_t)g.num_cus ? 4 : items >= (size_t)g.num_cus ? 96 : 0;
+    return rows && pairs >= rows * c.E ? kPrefillTileRows : kGemmTileRows;
 }
 
 void grouped_workspace_free() {
