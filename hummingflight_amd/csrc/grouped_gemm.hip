@@ -899,14 +899,33 @@ template <class Run>
 __device__ __forceinline__ void dynamic_items(const GemmArgs& a, const ItemRange& r, Run&& run) {
     const int t = threadIdx.x;
     __shared__ int next_item;
-    int probe = 0;  // thread 0: counters found spent, in probing order from this XCD's
-    auto grab = [&]() { return (int)atomicAdd(a.item_ctr + (r.xcd + probe) % r.nxcd, 1u); };
-    // Thread 0: the item of grab li, probing the next counters once one is spent; -1 when all are.
+    // Thread 0: bit i, counter (xcd + i) % nxcd is not known to be spent; it
+    // draws from the lowest.  Bit 8: the others have not been looked at yet.
+    unsigned open = 0x100u | ((1u << r.nxcd) - 1u);
+    auto ctr = [&](int i) { return a.item_ctr + (r.xcd + i) % r.nxcd; };
+    auto grab = [&]() { return (int)atomicAdd(ctr(__builtin_ctz(open)), 1u); };
+    // Thread 0: the item of grab li, going on to the next counters once one is
+    // spent; -1 when all are.  The first time, all counters are looked at
+    // together (one memory latency; a counter only grows, so a spent one stays
+    // so): at a launch's end every workgroup finds all of them spent, and one
+    // atomic after the other was the last thing the kernel waited for (64
+    // experts of 2048 x 1024, T = 1000: gate/up 226 -> 212-217 us).
     auto settle = [&](int li) {
         for (;;) {
-            const int x = (r.xcd + probe) % r.nxcd;
+            const int x = (r.xcd + __builtin_ctz(open)) % r.nxcd;
             if (li < xcd_items(r.deal(), x)) return xcd_item(r.deal(), x, li);
-            if (++probe >= r.nxcd) return -1;
+            open &= open - 1u;
+            if (open & 0x100u) {
+                int seen[8];
+#pragma unroll
+                for (int i = 1; i < 8; ++i)
+                    seen[i] = i < r.nxcd ? (int)__hip_atomic_load(ctr(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+                open = 0u;
+#pragma unroll
+                for (int i = 1; i < 8; ++i)
+                    if (i < r.nxcd && seen[i] < xcd_items(r.deal(), (r.xcd + i) % r.nxcd)) open |= 1u << i;
+            }
+            if (open == 0u) return -1;
             li = grab();
         }
     };
@@ -921,9 +940,9 @@ __device__ __forceinline__ void dynamic_items(const GemmArgs& a, const ItemRange
     while (item >= 0) {
         int li = 0;
         run(item, [&] {
-            if (t == 0 && probe < r.nxcd) li = grab();
+            if (t == 0 && open != 0u) li = grab();
         });
-        item = publish(t == 0 ? (probe < r.nxcd ? settle(li) : -1) : 0);
+        item = publish(t == 0 ? (open != 0u ? settle(li) : -1) : 0);
     }
 }
 
@@ -1652,8 +1671,14 @@ static hipError_t launch_shape(const GemmArgs& a, int blocks, hipStream_t s) {
         }
         return hipErrorInvalidValue;
     }
-    if (a.tile_rows == 192 && a.tile_cols == 64 * split_cb<EPI, 192>()) return launch_gemm_split<EPI, LOM, 192>(a, blocks, s);
-    if (a.tile_rows == 256 && a.tile_cols == 64 * split_cb<EPI, 256>()) return launch_gemm_split<EPI, LOM, 256>(a, blocks, s);
+    if constexpr (EPI != EPI_PARTIAL) {  // MoE GEMMs
+        if (a.tile_rows == 192 && a.tile_cols == 64 * split_cb<EPI, 192>())
+            return launch_gemm_split<EPI, LOM, 192>(a, blocks, s);
+    }
+    if constexpr (EPI != EPI_SCATTER) {  // one-group GEMMs
+        if (a.tile_rows == 256 && a.tile_cols == 64 * split_cb<EPI, 256>())
+            return launch_gemm_split<EPI, LOM, 256>(a, blocks, s);
+    }
     if (a.tile_rows == kGemmTileRows && a.tile_cols == GBN) return launch_gemm<EPI, LOM, 4>(a, blocks, s);
     return hipErrorInvalidValue;
 }
@@ -1682,8 +1707,7 @@ hipError_t launch_grouped_gemm(int epi, const GemmArgs& a, int blocks, hipStream
     // A second fixed matrix along N: split-kernel PARTIAL tiles that stay on
     // one side of the boundary.
     if (a.b_split && (epi != EPI_PARTIAL || a.b_tab || !a.b_fixed1 || a.b_split < 0 || a.b_split >= a.N ||
-                      (a.tile_rows != kPrefillTileRows && a.tile_rows != kDenseTileRows) ||
-                      a.b_split % a.tile_cols))
+                      a.tile_rows != kDenseTileRows || a.b_split % a.tile_cols))
         return hipErrorInvalidValue;
     switch (epi) {
         case EPI_PARTIAL: return launch_epi<EPI_PARTIAL>(a, blocks, s);

@@ -61,8 +61,8 @@ struct GemmArgs {
     const uint16_t* b_fixed0;
     const uint16_t* b_fixed1;
     int b_ld;                   // B row stride in elements
-    // PARTIAL with fixed B on the split kernel's tiles (tile_rows
-    // kPrefillTileRows or kDenseTileRows): output columns [b_split, N)
+    // PARTIAL with fixed B on the split kernel's 256-row tiles (tile_rows
+    // kDenseTileRows): output columns [b_split, N)
     // multiply rows (column - b_split) of b_fixed1, the columns before them
     // b_fixed0's (a gate / up pair as one [2 I, K] matrix; b_split a multiple
     // of the tile's columns).  0: b_fixed0 only.
