@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void gateup_t1_kernel(const float* __restrict_
         for (int r = 0; r < kk; ++r) ids.set(r, sm.sel[r]);
         if (blockIdx.x == 0 && (int)threadIdx.x < kk) {
             sel_io[threadIdx.x] = sm.sel[threadIdx.x];
-            selw_out[threadIdx.x] = sm.w[threadIdx.x];
+            selw_out[threadIdx.x] = select_weight(c, sm, kk, threadIdx.x);
         }
     } else {
         for (int r = 0; r < c.k; ++r) ids.set(r, sel_io[r]);

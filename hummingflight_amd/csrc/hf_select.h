@@ -89,7 +89,7 @@ struct SelectSmem {
     float gscore[kMaxGroups];
     int kept[kSelectMaxChunks];                // per chunk: its group is kept
     int sel[kMaxTopK];
-    float w[kMaxTopK];
+    float w[kMaxTopK];                         // the winners' unbiased scores
 };
 
 // This thread's score pairs (experts t, t + 256, ...), loaded ahead of other
@@ -116,7 +116,7 @@ __device__ __forceinline__ int select_chunk(int gs) {
 // Select k experts for one token from its score pairs [E] (fetched by
 // select_fetch).  Must be called by all 256 threads of the block (it
 // synchronises the block).  On return sm.sel[r] / sm.w[r] (r < k) hold the ids
-// in rank order and the final weights; the return value is k.
+// in rank order and their unbiased scores; the return value is k.
 __device__ __forceinline__ int select_block(const SelectRegs& regs, const Cfg& c, SelectSmem& sm) {
 #pragma clang fp contract(off)
     const int t = threadIdx.x;
@@ -209,18 +209,21 @@ __device__ __forceinline__ int select_block(const SelectRegs& regs, const Cfg& c
         }
     }
     __syncthreads();
-    if (t == 0) {
-        // moe_router.h:49-56: rank-order sum of the unbiased scores, normalise, scale.
-        float sum = 0.0f;
-        for (int r = 0; r < kk; ++r) sum = sum + sm.w[r];
-        for (int r = 0; r < kk; ++r) {
-            float wr = sm.w[r];
-            if (c.norm && sum > 0.0f) wr = wr / sum;
-            sm.w[r] = wr * c.scale;
-        }
-    }
-    __syncthreads();
     return kk;
+}
+
+// The final weight of rank t (t < k), after select_block: the rank-order sum
+// of the winners' unbiased scores, normalise, scale (moe_router.h:49-56).
+// Every rank's thread sums for itself, so that one division, not k of them
+// one after the other, follows the ranking; callers that need only the ids
+// leave it out.
+__device__ __forceinline__ float select_weight(const Cfg& c, const SelectSmem& sm, int kk, int t) {
+#pragma clang fp contract(off)
+    float sum = 0.0f;
+    for (int r = 0; r < kk; ++r) sum = sum + sm.w[r];
+    float wr = sm.w[t];
+    if (c.norm && sum > 0.0f) wr = wr / sum;
+    return wr * c.scale;
 }
 
 }  // namespace hf

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(const float2* __
     const int kk = select_block(regs, c, sm);
     if ((int)threadIdx.x < kk) {
         sel_idx[(size_t)tok * c.k + threadIdx.x] = sm.sel[threadIdx.x];
-        sel_w[(size_t)tok * c.k + threadIdx.x] = sm.w[threadIdx.x];
+        sel_w[(size_t)tok * c.k + threadIdx.x] = select_weight(c, sm, kk, threadIdx.x);
     }
 }
 
