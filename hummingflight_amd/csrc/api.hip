@@ -365,6 +365,12 @@ int hfmoe_register_layer(int layer, const hfmoe_layer_weights* w) {
     return HFMOE_OK;
 }
 
+// Two tokens go through the decode kernels one at a time: 0.225 against
+// 0.25-0.26 ms per layer at full shape (the grouped path's seven launches and
+// dispatch cost more than a second read of the few experts the two share);
+// from three tokens on the grouped path is as fast or faster.
+static bool tokenwise(int T) { return T <= env_int("HFMOE_TOKENWISE_MAX_T", 2); }
+
 int hfmoe_moe_forward(int layer, const float* x_dev, int32_t T, float* out_dev, void* stream) {
     return hfmoe_moe_forward_debug(layer, x_dev, T, out_dev, stream, nullptr);
 }
@@ -402,12 +408,8 @@ int hfmoe_moe_forward_debug(int layer, const float* x_dev, int32_t T, float* out
         return HFMOE_OK;
     }
     if (T == 1) return forward_t1(L, x_dev, out_dev, s, dbg);
-    // Two tokens go through the decode kernels one at a time: 0.225 against
-    // 0.25-0.26 ms per layer at full shape (the grouped path's seven launches
-    // and dispatch cost more than a second read of the few experts the two
-    // share); from three tokens on the grouped path is as fast or faster.  A
-    // debug call takes the grouped path, whose dispatch it reports.
-    if (!dbg && T <= env_int("HFMOE_TOKENWISE_MAX_T", 2)) {
+    // A debug call takes the grouped path, whose dispatch it reports.
+    if (!dbg && tokenwise(T)) {
         for (int t = 0; t < T; ++t) {
             rc = forward_t1(L, x_dev + (size_t)t * g.cfg.d, out_dev + (size_t)t * g.cfg.d, s, nullptr);
             if (rc) return rc;
@@ -479,14 +481,19 @@ int hfmoe_mlp_block(int layer, float* h_dev, int32_t T, void* stream) {
         return fail(HFMOE_ERR_INVALID_ARGUMENT, "hidden state must be 16-byte aligned");
     if (!g.ws.tmp) return fail(HFMOE_ERR_NOT_INITIALIZED, "workspace is not allocated");
     hipStream_t s = pick_stream(stream);
+    // A batch of an HBM-resident MoE layer: the norm and the residual add as
+    // part of the multi-token path's own kernels.
+    LayerState& L = it->second;
+    if (!L.dense && L.location == HFMOE_EXPERTS_DEVICE && g.gws.xh && T > 1 && !tokenwise(T))
+        return forward_grouped_block(L, h_dev, T, s);
     float* xn = g.ws.tmp;
     float* mo = g.ws.tmp + (size_t)T * g.cfg.d;
     Pending p;
     prof_begin(p, "rmsnorm", s);
-    hipError_t e = launch_rmsnorm(h_dev, it->second.norm_w, xn, T, g.cfg.d, g.cfg.eps, s);
+    hipError_t e = launch_rmsnorm(h_dev, L.norm_w, xn, T, g.cfg.d, g.cfg.eps, nullptr, s);
     prof_end(p, s);
     if (e != hipSuccess) return fail_hip(e, "rmsnorm launch");
-    rc = it->second.dense ? hfmoe_dense_mlp_forward(layer, xn, T, mo, s) : hfmoe_moe_forward(layer, xn, T, mo, s);
+    rc = L.dense ? hfmoe_dense_mlp_forward(layer, xn, T, mo, s) : hfmoe_moe_forward(layer, xn, T, mo, s);
     if (rc) return rc;
     prof_begin(p, "residual_add", s);
     e = launch_add_inplace(h_dev, mo, (size_t)T * g.cfg.d, s);

@@ -169,7 +169,7 @@ static int dense_fixed_forward(LayerState& L, int T, float* out, hipStream_t s) 
     gu.N = I;
     gu.a_hi = gw.xh;
     gu.a_lo = gw.xl;
-    gu.a_lo_flag = gw.lo_flag;
+    gu.a_lo_flag = gw.one_lo_flag();
     gu.b_fixed0 = L.dev.sg;
     gu.b_fixed1 = L.dev.su;
     gu.b_ld = c.d;
@@ -228,7 +228,9 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
     GroupedWorkspace& gw = g.gws;
     const int I = L.dense_inter;
     prof_begin(p, "split_x", s);
-    HF_CHECK_LAUNCH(launch_split_bf16(x, gw.xh, gw.xl, (size_t)T * c.d, gw.lo_flag, s), "split x");
+    HF_CHECK_LAUNCH(launch_clear_u32(gw.one_lo_flag(), 1, s), "flag clear");
+    prof_begin(p, "split_x", s);
+    HF_CHECK_LAUNCH(launch_split_bf16(x, gw.xh, gw.xl, (size_t)T * c.d, gw.one_lo_flag(), s), "split x");
     if (dense_fixed(T, I)) return dense_fixed_forward(L, T, out, s);
     // Layers too small for those tiles: past one 128-row M tile, the 256-row
     // tiles (HFMOE_DENSE_MIN_TOKENS).
@@ -243,7 +245,7 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
     gu.rows_total = T;
     gu.a_hi = gw.xh;
     gu.a_lo = gw.xl;
-    gu.a_lo_flag = gw.lo_flag;
+    gu.a_lo_flag = gw.one_lo_flag();
     gu.b_fixed0 = L.dev.sg;
     gu.b_fixed1 = L.dev.su;
     gu.b_ld = c.d;

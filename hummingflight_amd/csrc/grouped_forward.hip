@@ -3,9 +3,9 @@
 // The reference runs one token at a time (glm_forward.cpp:755-811); here all
 // T tokens go through the layer together, each expert's weights read once:
 //   1. x -> BF16 hi/lo halves (+ a device flag when any lo half is nonzero)
-//   2. router logits [T, E] by grouped GEMM with split-K, reduced in fixed order,
-//      then score pairs (sigmoid, sigmoid + bias)
-//   3. per-token selection (hf_select.h), one block per token
+//   2. router logits [T, E] by grouped GEMM with split-K
+//   3. per-token selection (hf_select.h), one block per token: the partials
+//      reduced in fixed order, score pairs (sigmoid, sigmoid + bias), ranking
 //   4. dispatch: stable counting sort of (token, rank) pairs by expert
 //   5. gate/up grouped GEMM over the routed groups plus the shared expert as
 //      one more group -> h (BF16 hi/lo, sorted rows)
@@ -128,6 +128,8 @@ int grouped_workspace_alloc() {
                         hipGetErrorString(e));
         }
     }
+    hipError_t e = hipMemset(w.lo_flag, 0, 256);  // zero between MoE calls
+    if (e != hipSuccess) return fail_hip(e, "hipMemset(flag)");
     return HFMOE_OK;
 }
 
@@ -150,16 +152,25 @@ static bool prefill_wide(int TR) {
     return TR == kPrefillTileRows && g.cfg.I % (kWideTileCols / 2) == 0 && env_int("HFMOE_PREFILL_WIDE", 1) != 0;
 }
 
-int grouped_route(LayerState& L, const float* x, int T, hipStream_t s) {
+// The flag of a MoE call's x is zero between calls (GroupedWorkspace): only
+// after one that failed half-way it is cleared here.
+static int grouped_flag_begin(hipStream_t s) {
+    GroupedWorkspace& w = g.gws;
+    if (w.lo_dirty) {
+        const hipError_t e = launch_clear_u32(w.lo_flag, 1, s);
+        if (e != hipSuccess) return fail_hip(e, "flag clear");
+    }
+    w.lo_dirty = true;
+    return HFMOE_OK;
+}
+
+// Routing of the T rows in gws.xh / xl.
+static int grouped_route_split(LayerState& L, int T, hipStream_t s) {
     const Cfg& c = g.cfg;
     GroupedWorkspace& w = g.gws;
     const int shared_rows = c.n_shared > 0 ? T : 0;
     const int TR = expert_tile_rows(T);
     Pending p;
-
-    prof_begin(p, "split_x", s);
-    HF_CHECK_LAUNCH(launch_split_bf16(x, w.xh, w.xl, (size_t)T * c.d, w.lo_flag, s), "split x");
-
     const int ks = router_ksplit(T);
     GemmArgs r{};
     r.K = c.d;
@@ -178,11 +189,8 @@ int grouped_route(LayerState& L, const float* x, int T, hipStream_t s) {
     r.ksplit = ks;
     prof_begin(p, "router_gemm", s);
     HF_CHECK_LAUNCH(launch_grouped_gemm(EPI_PARTIAL, r, gemm_blocks(kGemmTileRows), s), "router gemm");
-    prof_begin(p, "router_reduce", s);
-    HF_CHECK_LAUNCH(launch_router_reduce(w.part, ks, T, c.E, L.dev.bias, g.ws.logits, g.ws.scores, s),
-                    "router reduce");
     prof_begin(p, "select", s);
-    HF_CHECK_LAUNCH(launch_select(g.ws.scores, T, c, g.ws.idx, g.ws.wts, s), "select");
+    HF_CHECK_LAUNCH(launch_router_select(w.part, ks, T, L.dev.bias, c, g.ws.logits, g.ws.idx, g.ws.wts, s), "select");
     prof_begin(p, "dispatch", s);
     TileList tl{TR, w.tile_expert, w.tile_row0, w.ntiles}, tl_gu{};
     w.wide = prefill_wide(TR);
@@ -191,6 +199,16 @@ int grouped_route(LayerState& L, const float* x, int T, hipStream_t s) {
                                     w.row_token, w.chunk_hist, TR == kPrefillTileRows ? w.item_ctr : nullptr, s),
                     "dispatch");
     return HFMOE_OK;
+}
+
+int grouped_route(LayerState& L, const float* x, int T, hipStream_t s) {
+    GroupedWorkspace& w = g.gws;
+    Pending p;
+    int rc = grouped_flag_begin(s);
+    if (rc) return rc;
+    prof_begin(p, "split_x", s);
+    HF_CHECK_LAUNCH(launch_split_bf16(x, w.xh, w.xl, (size_t)T * g.cfg.d, w.lo_flag, s), "split x");
+    return grouped_route_split(L, T, s);
 }
 
 int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s) {
@@ -274,12 +292,15 @@ int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s) {
     return HFMOE_OK;
 }
 
-int grouped_combine(int T, float* out, hipStream_t s) {
+int grouped_combine(int T, const float* residual, float* out, hipStream_t s) {
     const Cfg& c = g.cfg;
     const int P = T * c.k;
     Pending p;
     prof_begin(p, "combine", s);
-    HF_CHECK_LAUNCH(launch_combine(g.ws.wts, g.gws.y, T, c.k, c.d, c.n_shared > 0 ? P : -1, out, s), "combine");
+    HF_CHECK_LAUNCH(launch_combine(g.ws.wts, g.gws.y, T, c.k, c.d, c.n_shared > 0 ? P : -1, residual, out,
+                                   g.gws.lo_flag, s),
+                    "combine");
+    g.gws.lo_dirty = false;
     return HFMOE_OK;
 }
 
@@ -288,8 +309,25 @@ int forward_grouped(LayerState& L, const float* x, int T, float* out, hipStream_
     if (!g.gws.xh) return forward_tokenwise(L, x, T, out, s, dbg);
     int rc = grouped_route(L, x, T, s);
     if (!rc) rc = grouped_experts(L.dev.etab, T, s);
-    if (!rc) rc = grouped_combine(T, out, s);
+    if (!rc) rc = grouped_combine(T, nullptr, out, s);
     return rc ? rc : copy_debug(dbg, T, s);
+}
+
+// The norm writes the halves that the GEMMs read and the combine adds to the
+// residual stream: of eleven launches and 32 bytes per element of h read and
+// written around the GEMMs seven and 16 are left (GLM-5.2 layer T = 7 650 ->
+// 643 us, 509 3296 -> 3270; same bits).
+int forward_grouped_block(LayerState& L, float* h, int T, hipStream_t s) {
+    const Cfg& c = g.cfg;
+    GroupedWorkspace& w = g.gws;
+    Pending p;
+    int rc = grouped_flag_begin(s);
+    if (rc) return rc;
+    prof_begin(p, "rmsnorm", s);
+    HF_CHECK_LAUNCH(launch_rmsnorm_split(h, L.norm_w, w.xh, w.xl, T, c.d, c.eps, w.lo_flag, s), "rmsnorm launch");
+    rc = grouped_route_split(L, T, s);
+    if (!rc) rc = grouped_experts(L.dev.etab, T, s);
+    return rc ? rc : grouped_combine(T, h, h, s);
 }
 
 }  // namespace hf

@@ -1391,9 +1391,12 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void grouped_gemm_fixed_kernel(
 
 // out[t] = (sum_r w[t, r] * y[t*k + r]) + y[shared_row0 + t] (when shared_row0 >= 0):
 // the weighted merge in rank order, then the shared expert (glm_forward.cpp:639-640, 658-660).
+// residual (may be out itself): added last, out = residual + that
+// (glm_forward.cpp:795).  clear: one word zeroed for the next call.
 __global__ void combine_kernel(const float* __restrict__ wts, const float* __restrict__ y, int T, int k,
-                               int d, int shared_row0, float* __restrict__ out) {
+                               int d, int shared_row0, const float* residual, float* out, unsigned* clear) {
     const size_t i4 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i4 == 0) *clear = 0u;
     const int d4 = d >> 2;
     if (i4 >= (size_t)T * d4) return;
     const int t = (int)(i4 / d4), n4 = (int)(i4 % d4);
@@ -1414,6 +1417,10 @@ __global__ void combine_kernel(const float* __restrict__ wts, const float* __res
         m.y += v.y;
         m.z += v.z;
         m.w += v.w;
+    }
+    if (residual) {
+        const float4 h = reinterpret_cast<const float4*>(residual)[i4];
+        m = make_float4(h.x + m.x, h.y + m.y, h.z + m.z, h.w + m.w);
     }
     reinterpret_cast<float4*>(out)[i4] = m;
 }
@@ -1455,7 +1462,8 @@ __global__ void split_bf16_kernel(const float* __restrict__ x, uint16_t* __restr
         lo[i] = l;
         nz |= (l & 0x7FFF) != 0;
     }
-    // A plain store: the flag only goes from 0 (cleared by an earlier kernel)
+    // A plain store: the flag only goes from 0 (cleared by an earlier kernel,
+    // see launch_split_bf16)
     // to 1 and is read by later kernels; with FP32 activations every
     // wavefront sets it, and as many device-scope atomics on one address
     // serialise at the memory (x split of 4096 x 6144: 199 -> 37 us).
@@ -1556,28 +1564,6 @@ __global__ void clear_u32_kernel(unsigned* p, int n) {
 
 hipError_t launch_clear_u32(unsigned* p, int n, hipStream_t s) {
     return launch(clear_u32_kernel, dim3((n + 63) / 64), dim3(64), 0, s, p, n);
-}
-
-// Router logits from split-K partials (summed in split order) and score pairs.
-__global__ void router_reduce_kernel(const float* __restrict__ part, int ksplit, int T, int E,
-                                     const float* __restrict__ bias, float* __restrict__ logits,
-                                     float2* __restrict__ scores) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= T * E) return;
-    const size_t st = (size_t)T * E;
-    // Eight partials loaded at a time, summed in split order.
-    float s = 0.0f;
-    int q = 0;
-    for (; q + 8 <= ksplit; q += 8) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = __builtin_nontemporal_load(part + (q + u) * st + i);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; q < ksplit; ++q) s += part[q * st + i];
-    logits[i] = s;
-    scores[i] = score_pair(s, bias, i % E);
 }
 
 template <int EPI, int LOM, int WAVES>
@@ -1718,27 +1704,17 @@ hipError_t launch_grouped_gemm(int epi, const GemmArgs& a, int blocks, hipStream
 }
 
 hipError_t launch_combine(const float* wts, const float* y, int T, int k, int d, int shared_row0,
-                          float* out, hipStream_t s) {
+                          const float* residual, float* out, unsigned* clear, hipStream_t s) {
     const size_t n4 = (size_t)T * (d / 4);
     return launch(combine_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, wts, y, T, k, d,
-                  shared_row0, out);
+                  shared_row0, residual, out, clear);
 }
 
 hipError_t launch_split_bf16(const float* x, uint16_t* hi, uint16_t* lo, size_t n, unsigned* flag,
                              hipStream_t s) {
-    // flag[0]: x has a nonzero lo half (set below).
-    hipError_t e = launch(clear_u32_kernel, dim3(1), dim3(64), 0, s, flag, 1);
-    if (e != hipSuccess) return e;
     size_t blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
     return launch(split_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, hi, lo, n, flag);
-}
-
-hipError_t launch_router_reduce(const float* part, int ksplit, int T, int E, const float* bias,
-                                float* logits, float2* scores, hipStream_t s) {
-    const int n = T * E;
-    return launch(router_reduce_kernel, dim3((n + 255) / 256), dim3(256), 0, s, part, ksplit, T, E,
-                  bias, logits, scores);
 }
 
 }  // namespace hf

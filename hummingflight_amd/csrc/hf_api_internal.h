@@ -46,7 +46,12 @@ struct GroupedWorkspace {
     bool wide = false;              // the last dispatch wrote that list (the GEMMs after it take the wide tiles)
     int* chunk_hist = nullptr;   // [kDispatchMaxChunks, E] dispatch chunk counts / first slots
     unsigned* item_ctr = nullptr;  // [kItemCounters] prefill GEMM work counters (zeroed by the dispatch)
-    unsigned int* lo_flag = nullptr;  // [0] x has a nonzero BF16 lo half
+    // x has a nonzero BF16 lo half: of a MoE call (zero between calls, the
+    // combine clears it; lo_dirty: a call ended before its combine), and, a
+    // 128-byte line further, of a dense or LM-head call (cleared by each).
+    unsigned int* lo_flag = nullptr;
+    bool lo_dirty = false;
+    unsigned int* one_lo_flag() const { return lo_flag + 32; }
     uint16_t* xh = nullptr;      // [maxT, d] x BF16 hi (token order)
     uint16_t* xl = nullptr;      // [maxT, d] x BF16 lo
     uint16_t* hh = nullptr;      // [rows, I] h hi (sorted rows)
@@ -206,13 +211,16 @@ int copy_debug(const hfmoe_route_debug* dbg, int T, hipStream_t s);
 // grouped_forward.hip
 int forward_grouped(LayerState& L, const float* x, int T, float* out, hipStream_t s,
                     const hfmoe_route_debug* dbg);
+// h += MoE(RMSNorm(h)) over the multi-token path (grouped workspace allocated).
+int forward_grouped_block(LayerState& L, float* h, int T, hipStream_t s);
 // The three phases of forward_grouped (multi-token path, grouped workspace
 // allocated): routing (x split, router, selection, dispatch), the expert
 // gate/up and down GEMMs of the groups whose etab entries are not null (3 per
-// group, E + 1 groups, the shared expert last), and the weighted combine.
+// group, E + 1 groups, the shared expert last), and the weighted combine
+// (added to residual when given, which may be out).
 int grouped_route(LayerState& L, const float* x, int T, hipStream_t s);
 int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s);
-int grouped_combine(int T, float* out, hipStream_t s);
+int grouped_combine(int T, const float* residual, float* out, hipStream_t s);
 int grouped_tile_rows(int T);
 int grouped_workspace_alloc();
 void grouped_workspace_free();
@@ -233,8 +241,13 @@ int streamed_forward_batch(int layer, LayerState& L, const float* x, int T, floa
                            const hfmoe_route_debug* dbg);
 void stream_pool_release();
 // misc kernels
+// clear (may be null): one word zeroed.
 hipError_t launch_rmsnorm(const float* h, const uint16_t* w, float* out, int T, int d, float eps,
-                          hipStream_t s);
+                          unsigned* clear, hipStream_t s);
+// The normalised rows as BF16 hi / lo halves; *flag (0 before) = 1 when any lo
+// half is nonzero.
+hipError_t launch_rmsnorm_split(const float* h, const uint16_t* w, uint16_t* hi, uint16_t* lo, int T, int d, float eps,
+                                unsigned* flag, hipStream_t s);
 hipError_t launch_add_inplace(float* dst, const float* src, size_t n, hipStream_t s);
 hipError_t launch_copy_f32(const float* src, float* dst, size_t n, hipStream_t s);
 hipError_t launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStream_t s);

@@ -116,13 +116,16 @@ hipError_t launch_sum_splits(const float* part, int ks, size_t n, float* out, hi
 // [T][I] (I a multiple of 4).
 hipError_t launch_swiglu_splits(const float* part, int ks, int T, int I, uint16_t* h_hi, uint16_t* h_lo,
                                 hipStream_t s);
+// x FP32 -> BF16 hi / lo; *flag = 1 when any lo half is nonzero.  The flag must
+// be 0 before: an earlier kernel clears it (the combine of the MoE call before,
+// a norm or launch_clear_u32), as a launch of its own costs as much as the
+// split of a short batch.
 hipError_t launch_split_bf16(const float* x, uint16_t* hi, uint16_t* lo, size_t n, unsigned* flag,
                              hipStream_t s);
-// out[t] = sum_r wts[t, r] * y[t*k + r] (+ y[shared_row0 + t] when shared_row0 >= 0); d % 4 == 0.
+// out[t] = sum_r wts[t, r] * y[t*k + r] (+ y[shared_row0 + t] when shared_row0 >= 0)
+// (residual[t] + that, when given; residual may be out); d % 4 == 0.  *clear = 0.
 hipError_t launch_combine(const float* wts, const float* y, int T, int k, int d, int shared_row0,
-                          float* out, hipStream_t s);
-hipError_t launch_router_reduce(const float* part, int ksplit, int T, int E, const float* bias,
-                                float* logits, float2* scores, hipStream_t s);
+                          const float* residual, float* out, unsigned* clear, hipStream_t s);
 // Stable counting sort of the T*k (token, rank) pairs by expert plus the M-tile
 // list (tile_rows rows per tile) of the grouped GEMM.  With shared_rows > 0 a
 // group E of shared_rows rows (sorted rows T*k + t <- token t) follows the

@@ -62,6 +62,11 @@ hipError_t launch_router_logits(const float* x, int T, const LayerDev& L, const 
 hipError_t launch_select(const float2* scores, int T, const Cfg& c, int* sel_idx, float* sel_w,
                          hipStream_t s);
 
+// The same from the router GEMM's split-K partials [ksplit][T][E], summed in
+// split order into logits [T, E].
+hipError_t launch_router_select(const float* part, int ksplit, int T, const float* bias, const Cfg& c, float* logits,
+                                int* sel_idx, float* sel_w, hipStream_t s);
+
 // expert_gemv.hip -- decode (T = 1) expert SwiGLU.
 // Slots 0..k-1 are the selected experts (sel_idx), slots k.. are the shared
 // expert's n_shared slices of I rows.  h: FP32 [nslots, I].

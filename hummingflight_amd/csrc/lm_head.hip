@@ -254,8 +254,9 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     float* xn = g.ws.tmp;  // [T, d]
     Pending p;
     prof_begin(p, "lm_norm", s);
-    HF_CHECK_LAUNCH(launch_rmsnorm(h, L.norm, xn, T, c.d, c.eps, s), "final norm");
     const bool gemm = T > 1 && g.gws.xh && c.d % kGemmTileK == 0;
+    HF_CHECK_LAUNCH(launch_rmsnorm(h, L.norm, xn, T, c.d, c.eps, gemm ? g.gws.one_lo_flag() : nullptr, s),
+                    "final norm");
     if (!gemm) {
         const int grid = lm_call_grid();
         for (int t = 0; t < T; ++t) {
@@ -274,14 +275,14 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     }
     GroupedWorkspace& gw = g.gws;
     prof_begin(p, "split_x", s);
-    HF_CHECK_LAUNCH(launch_split_bf16(xn, gw.xh, gw.xl, (size_t)T * c.d, gw.lo_flag, s), "split x");
+    HF_CHECK_LAUNCH(launch_split_bf16(xn, gw.xh, gw.xl, (size_t)T * c.d, gw.one_lo_flag(), s), "split x");
     GemmArgs a{};
     a.K = c.d;
     a.N = L.vocab;
     a.rows_total = T;
     a.a_hi = gw.xh;
     a.a_lo = gw.xl;
-    a.a_lo_flag = gw.lo_flag;
+    a.a_lo_flag = gw.one_lo_flag();
     a.b_fixed0 = L.w;
     a.b_ld = c.d;
     a.out_f32 = logits;

@@ -11,8 +11,10 @@ namespace hf {
 constexpr int kNormThreads = 1024;
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float* __restrict__ h,
                                                                const uint16_t* __restrict__ w,
-                                                               float* __restrict__ out, int d, float eps) {
+                                                               float* __restrict__ out, int d, float eps,
+                                                               unsigned* __restrict__ clear) {
     __shared__ float red[kNormThreads / 64];
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0u;
     const float* x = h + (size_t)blockIdx.x * d;
     float* y = out + (size_t)blockIdx.x * d;
     const bool vec = (d & 3) == 0;
@@ -49,6 +51,58 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float* __re
     } else {
         for (int i = threadIdx.x; i < d; i += kNormThreads) y[i] = x[i] * r * wt(i);
     }
+}
+
+// The same for d a multiple of 4, straight to the BF16 hi / lo halves that the
+// multi-token GEMMs read (hi = RNE(y), lo = RNE(y - hi), as split_bf16_kernel;
+// *flag = 1 when any lo half is nonzero): neither the FP32 rows nor a launch
+// between the norm and the GEMMs.
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_split_kernel(const float* __restrict__ h,
+                                                                     const uint16_t* __restrict__ w,
+                                                                     uint16_t* __restrict__ hi,
+                                                                     uint16_t* __restrict__ lo, int d, float eps,
+                                                                     unsigned* __restrict__ flag) {
+#pragma clang fp contract(off)  // lo is what the rounded y leaves, not the exact product
+    __shared__ float red[kNormThreads / 64];
+    const size_t row = (size_t)blockIdx.x * d;
+    float4 v[2];
+    float sq = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int i = 4 * (threadIdx.x + j * kNormThreads);
+        v[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (i < d) v[j] = *reinterpret_cast<const float4*>(h + row + i);
+        sq = fmaf(v[j].x, v[j].x, sq);
+        sq = fmaf(v[j].y, v[j].y, sq);
+        sq = fmaf(v[j].z, v[j].z, sq);
+        sq = fmaf(v[j].w, v[j].w, sq);
+    }
+    sq = wave_sum(sq);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sq;
+    __syncthreads();
+    float tot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kNormThreads / 64; ++i) tot += red[i];
+    const float r = 1.0f / sqrtf(tot / (float)d + eps);
+    auto wt = [&](int i) { return w ? __uint_as_float((uint32_t)w[i] << 16) : 1.0f; };
+    bool nz = false;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int i = 4 * (threadIdx.x + j * kNormThreads);
+        if (i < d) {
+            const float y[4] = {v[j].x * r * wt(i), v[j].y * r * wt(i + 1), v[j].z * r * wt(i + 2), v[j].w * r * wt(i + 3)};
+            uint32_t hw[4], lw[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                hw[q] = f32_to_bf16(y[q]);
+                lw[q] = f32_to_bf16(y[q] - __uint_as_float(hw[q] << 16));
+                nz |= (lw[q] & 0x7FFFu) != 0;
+            }
+            *reinterpret_cast<uint2*>(hi + row + i) = make_uint2(hw[0] | (hw[1] << 16), hw[2] | (hw[3] << 16));
+            *reinterpret_cast<uint2*>(lo + row + i) = make_uint2(lw[0] | (lw[1] << 16), lw[2] | (lw[3] << 16));
+        }
+    }
+    if (__ballot(nz) != 0ull && (threadIdx.x & 63) == 0) *flag = 1u;
 }
 
 __global__ void add_inplace_kernel(float* __restrict__ dst, const float* __restrict__ src, size_t n) {
@@ -118,9 +172,15 @@ hipError_t launch_copy_u64(const uint64_t* src, uint64_t* dst, size_t n, hipStre
 }
 
 hipError_t launch_rmsnorm(const float* h, const uint16_t* w, float* out, int T, int d, float eps,
-                          hipStream_t s) {
+                          unsigned* clear, hipStream_t s) {
     if (d > 8 * kNormThreads) return hipErrorInvalidValue;
-    return launch(rmsnorm_kernel, dim3(T), dim3(kNormThreads), 0, s, h, w, out, d, eps);
+    return launch(rmsnorm_kernel, dim3(T), dim3(kNormThreads), 0, s, h, w, out, d, eps, clear);
+}
+
+hipError_t launch_rmsnorm_split(const float* h, const uint16_t* w, uint16_t* hi, uint16_t* lo, int T, int d, float eps,
+                                unsigned* flag, hipStream_t s) {
+    if (d > 8 * kNormThreads || d % 4) return hipErrorInvalidValue;
+    return launch(rmsnorm_split_kernel, dim3(T), dim3(kNormThreads), 0, s, h, w, hi, lo, d, eps, flag);
 }
 
 hipError_t launch_add_inplace(float* dst, const float* src, size_t n, hipStream_t s) {

@@ -364,7 +364,7 @@ int streamed_forward_batch(int layer, LayerState& L, const float* x, int T, floa
         if (rc) return rc;
         claimed.push_back(slot);
     }
-    rc = grouped_combine(T, out, s);
+    rc = grouped_combine(T, nullptr, out, s);
     return rc ? rc : copy_debug(dbg, T, s);
 }
 
