@@ -428,8 +428,14 @@ int hfmoe_moe_forward_bf16(int layer, const uint16_t* x_dev, int32_t T, float* o
     if (!x_dev) return fail(HFMOE_ERR_INVALID_ARGUMENT, "null activation pointer");
     if (reinterpret_cast<uintptr_t>(x_dev) & 15) return fail(HFMOE_ERR_INVALID_ARGUMENT, "x must be 16-byte aligned");
     if (!g.ws.tmp) return fail(HFMOE_ERR_NOT_INITIALIZED, "workspace is not allocated");
-    // x widened to FP32 (exactly) in the workspace's [max_tokens, d] scratch
-    // rows, then the FP32 forward on the same stream.
+    // A batch of an HBM-resident MoE layer: the multi-token path's GEMMs take
+    // BF16 x as it is.  (Anything else, and every error, as in the FP32 call.)
+    auto it = g.layers.find(layer);
+    if (it != g.layers.end() && !it->second.dense && it->second.location == HFMOE_EXPERTS_DEVICE && g.gws.xh && T > 1 &&
+        !tokenwise(T) && out_dev && !(reinterpret_cast<uintptr_t>(out_dev) & 15))
+        return forward_grouped_bf16(it->second, x_dev, T, out_dev, pick_stream(stream));
+    // Else x widened to FP32 (exactly) in the workspace's [max_tokens, d]
+    // scratch rows, then the FP32 forward on the same stream.
     hipError_t e = launch_bf16_to_f32(x_dev, g.ws.tmp, (size_t)T * g.cfg.d, pick_stream(stream));
     if (e != hipSuccess) return fail_hip(e, "x BF16 -> FP32");
     return hfmoe_moe_forward_debug(layer, g.ws.tmp, T, out_dev, stream, nullptr);
@@ -490,7 +496,7 @@ int hfmoe_mlp_block(int layer, float* h_dev, int32_t T, void* stream) {
     float* mo = g.ws.tmp + (size_t)T * g.cfg.d;
     Pending p;
     prof_begin(p, "rmsnorm", s);
-    hipError_t e = launch_rmsnorm(h_dev, L.norm_w, xn, T, g.cfg.d, g.cfg.eps, nullptr, s);
+    hipError_t e = launch_rmsnorm(h_dev, L.norm_w, xn, T, g.cfg.d, g.cfg.eps, s);
     prof_end(p, s);
     if (e != hipSuccess) return fail_hip(e, "rmsnorm launch");
     rc = L.dense ? hfmoe_dense_mlp_forward(layer, xn, T, mo, s) : hfmoe_moe_forward(layer, xn, T, mo, s);

@@ -192,8 +192,10 @@ static int dense_fixed_forward(LayerState& L, int T, float* out, hipStream_t s) 
     dn.b_fixed0 = L.dev.sd;
     dn.b_ld = I;
     dn.out_f32 = pl.ksplit > 1 ? w.part : out;
+    dn.clear = gw.one_lo_flag();  // gate/up, its reader, is done
     prof_begin(p, "dense_down_gemm", s);
     HF_CHECK_LAUNCH(launch_fixed_gemm(EPI_PARTIAL, false, 4, dn, blocks, s), "dense down gemm");
+    gw.one_dirty = false;
     if (pl.ksplit > 1) {
         prof_begin(p, "dense_down_sum", s);
         HF_CHECK_LAUNCH(launch_sum_splits(w.part, pl.ksplit, (size_t)T * c.d, out, s), "dense down split sum");
@@ -227,8 +229,8 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
     }
     GroupedWorkspace& gw = g.gws;
     const int I = L.dense_inter;
-    prof_begin(p, "split_x", s);
-    HF_CHECK_LAUNCH(launch_clear_u32(gw.one_lo_flag(), 1, s), "flag clear");
+    const int rc = lo_flag_begin(gw.one_lo_flag(), gw.one_dirty, s);
+    if (rc) return rc;
     prof_begin(p, "split_x", s);
     HF_CHECK_LAUNCH(launch_split_bf16(x, gw.xh, gw.xl, (size_t)T * c.d, gw.one_lo_flag(), s), "split x");
     if (dense_fixed(T, I)) return dense_fixed_forward(L, T, out, s);
@@ -304,6 +306,8 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
     dn.by_ntile = by_ntile;
     prof_begin(p, "dense_down_gemm", s);
     HF_CHECK_LAUNCH(launch_grouped_gemm(EPI_PARTIAL, dn, gemm_blocks(TR), s), "dense down gemm");
+    HF_CHECK_LAUNCH(launch_clear_u32(gw.one_lo_flag(), 1, s), "flag clear");
+    gw.one_dirty = false;
     if (dn.ksplit > 1) {
         prof_begin(p, "dense_down_sum", s);
         HF_CHECK_LAUNCH(launch_sum_splits(w.part, dn.ksplit, (size_t)T * c.d, out, s), "dense down split sum");

@@ -152,20 +152,17 @@ static bool prefill_wide(int TR) {
     return TR == kPrefillTileRows && g.cfg.I % (kWideTileCols / 2) == 0 && env_int("HFMOE_PREFILL_WIDE", 1) != 0;
 }
 
-// The flag of a MoE call's x is zero between calls (GroupedWorkspace): only
-// after one that failed half-way it is cleared here.
-static int grouped_flag_begin(hipStream_t s) {
-    GroupedWorkspace& w = g.gws;
-    if (w.lo_dirty) {
-        const hipError_t e = launch_clear_u32(w.lo_flag, 1, s);
+int lo_flag_begin(unsigned* flag, bool& dirty, hipStream_t s) {
+    if (dirty) {
+        const hipError_t e = launch_clear_u32(flag, 1, s);
         if (e != hipSuccess) return fail_hip(e, "flag clear");
     }
-    w.lo_dirty = true;
+    dirty = true;
     return HFMOE_OK;
 }
 
-// Routing of the T rows in gws.xh / xl.
-static int grouped_route_split(LayerState& L, int T, hipStream_t s) {
+// Routing of T rows split into x_hi and gws.xl.
+static int grouped_route_split(LayerState& L, const uint16_t* x_hi, int T, hipStream_t s) {
     const Cfg& c = g.cfg;
     GroupedWorkspace& w = g.gws;
     const int shared_rows = c.n_shared > 0 ? T : 0;
@@ -180,7 +177,7 @@ static int grouped_route_split(LayerState& L, int T, hipStream_t s) {
     r.n_tiles = (c.E + 127) / 128;
     r.m_tiles = (T + kGemmTileRows - 1) / kGemmTileRows;
     r.rows_total = T;
-    r.a_hi = w.xh;
+    r.a_hi = x_hi;
     r.a_lo = w.xl;
     r.a_lo_flag = w.lo_flag;
     r.b_fixed0 = L.dev.router;
@@ -204,14 +201,14 @@ static int grouped_route_split(LayerState& L, int T, hipStream_t s) {
 int grouped_route(LayerState& L, const float* x, int T, hipStream_t s) {
     GroupedWorkspace& w = g.gws;
     Pending p;
-    int rc = grouped_flag_begin(s);
+    int rc = lo_flag_begin(w.lo_flag, w.lo_dirty, s);
     if (rc) return rc;
     prof_begin(p, "split_x", s);
     HF_CHECK_LAUNCH(launch_split_bf16(x, w.xh, w.xl, (size_t)T * g.cfg.d, w.lo_flag, s), "split x");
-    return grouped_route_split(L, T, s);
+    return grouped_route_split(L, w.xh, T, s);
 }
 
-int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s) {
+int grouped_experts(const uint16_t* const* etab, const uint16_t* x_hi, int T, hipStream_t s) {
     const Cfg& c = g.cfg;
     GroupedWorkspace& w = g.gws;
     const int P = T * c.k;
@@ -240,7 +237,7 @@ int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s) {
     }
     gu.group_end = w.offsets + 1;
     gu.rows_total = P + shared_rows;
-    gu.a_hi = w.xh;
+    gu.a_hi = x_hi;
     gu.a_lo = w.xl;
     gu.a_lo_flag = w.lo_flag;
     gu.a_rowmap = w.row_token;
@@ -308,9 +305,21 @@ int forward_grouped(LayerState& L, const float* x, int T, float* out, hipStream_
                     const hfmoe_route_debug* dbg) {
     if (!g.gws.xh) return forward_tokenwise(L, x, T, out, s, dbg);
     int rc = grouped_route(L, x, T, s);
-    if (!rc) rc = grouped_experts(L.dev.etab, T, s);
+    if (!rc) rc = grouped_experts(L.dev.etab, g.gws.xh, T, s);
     if (!rc) rc = grouped_combine(T, nullptr, out, s);
     return rc ? rc : copy_debug(dbg, T, s);
+}
+
+int forward_grouped_bf16(LayerState& L, const uint16_t* x, int T, float* out, hipStream_t s) {
+    GroupedWorkspace& w = g.gws;
+    Pending p;
+    int rc = lo_flag_begin(w.lo_flag, w.lo_dirty, s);
+    if (rc) return rc;
+    prof_begin(p, "split_x", s);
+    HF_CHECK_LAUNCH(launch_bf16_lo(x, w.xl, (size_t)T * g.cfg.d, w.lo_flag, s), "x lo halves");
+    rc = grouped_route_split(L, x, T, s);
+    if (!rc) rc = grouped_experts(L.dev.etab, x, T, s);
+    return rc ? rc : grouped_combine(T, nullptr, out, s);
 }
 
 // The norm writes the halves that the GEMMs read and the combine adds to the
@@ -321,12 +330,12 @@ int forward_grouped_block(LayerState& L, float* h, int T, hipStream_t s) {
     const Cfg& c = g.cfg;
     GroupedWorkspace& w = g.gws;
     Pending p;
-    int rc = grouped_flag_begin(s);
+    int rc = lo_flag_begin(w.lo_flag, w.lo_dirty, s);
     if (rc) return rc;
     prof_begin(p, "rmsnorm", s);
     HF_CHECK_LAUNCH(launch_rmsnorm_split(h, L.norm_w, w.xh, w.xl, T, c.d, c.eps, w.lo_flag, s), "rmsnorm launch");
-    rc = grouped_route_split(L, T, s);
-    if (!rc) rc = grouped_experts(L.dev.etab, T, s);
+    rc = grouped_route_split(L, w.xh, T, s);
+    if (!rc) rc = grouped_experts(L.dev.etab, w.xh, T, s);
     return rc ? rc : grouped_combine(T, h, h, s);
 }
 

@@ -1368,6 +1368,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 1) void grouped_gemm_fixed_kernel(
     const int t = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const bool use_lo = LOM == kLoAlways || *a.a_lo_flag != 0u;
+    if (a.clear && blockIdx.x == 0 && t == 0) *a.clear = 0u;
     const int total = a.m_tiles * a.n_tiles * a.ksplit;
     const int nxcd = gridDim.x >= 8 ? 8 : 1;
     const int xcd = blockIdx.x % nxcd;
@@ -1625,7 +1626,7 @@ hipError_t launch_fixed_gemm(int epi, bool pair, int cb, const GemmArgs& a, int 
         (size_t)a.m_tiles * a.tile_rows < (size_t)a.rows_total ||
         (size_t)(a.m_tiles - 1) * a.tile_rows >= (size_t)a.rows_total || a.N < fixed_tile_cols(cb, sw) ||
         (size_t)a.n_tiles * fixed_tile_cols(cb, sw) < (size_t)a.N || (sw && (a.N % 4 || !a.b_fixed1)) ||
-        (epi == EPI_SWIGLU && a.ksplit != 1) || blocks < 1 || (size_t)a.N * (size_t)a.b_ld * 2 >= lim ||
+        (epi == EPI_SWIGLU && a.ksplit != 1) || (a.clear && a.clear == a.a_lo_flag) || blocks < 1 || (size_t)a.N * (size_t)a.b_ld * 2 >= lim ||
         (size_t)a.rows_total * (size_t)a.K * 2 >= lim)
         return hipErrorInvalidValue;
     const bool flag = a.a_lo_flag != nullptr;

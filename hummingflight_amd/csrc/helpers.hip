@@ -174,7 +174,8 @@ int hfmoe_argmax_rows(const float* x_dev, int32_t T, int32_t n, int32_t* best_de
     if (!x_dev || !best_dev || n <= 0 || T < 0)
         return fail(HFMOE_ERR_INVALID_ARGUMENT, "argmax: null buffer or n <= 0");
     if (T == 0) return HFMOE_OK;
-    hipError_t e = launch_row_argmax(x_dev, T, n, reinterpret_cast<int*>(best_dev), pick_stream(stream));
+    hipError_t e = launch_row_argmax(x_dev, T, n, reinterpret_cast<int*>(best_dev), nullptr,
+                                     pick_stream(stream));
     return e == hipSuccess ? HFMOE_OK : fail_hip(e, "argmax launch");
 }
 
@@ -236,7 +237,7 @@ int hfmoe_argmax(const float* x_host, int n, int32_t* best) {
     hipError_t e = hipMalloc(&x.p, 4 * (size_t)n);
     if (e == hipSuccess) e = hipMalloc(&o.p, sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(x.p, x_host, 4 * (size_t)n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = launch_row_argmax(static_cast<const float*>(x.p), 1, n, static_cast<int*>(o.p), g.stream);
+    if (e == hipSuccess) e = launch_row_argmax(static_cast<const float*>(x.p), 1, n, static_cast<int*>(o.p), nullptr, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
     if (e == hipSuccess) e = hipMemcpy(best, o.p, sizeof(int), hipMemcpyDeviceToHost);
     return e == hipSuccess ? HFMOE_OK : fail_hip(e, "argmax");

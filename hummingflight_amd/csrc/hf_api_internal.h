@@ -46,11 +46,11 @@ struct GroupedWorkspace {
     bool wide = false;              // the last dispatch wrote that list (the GEMMs after it take the wide tiles)
     int* chunk_hist = nullptr;   // [kDispatchMaxChunks, E] dispatch chunk counts / first slots
     unsigned* item_ctr = nullptr;  // [kItemCounters] prefill GEMM work counters (zeroed by the dispatch)
-    // x has a nonzero BF16 lo half: of a MoE call (zero between calls, the
-    // combine clears it; lo_dirty: a call ended before its combine), and, a
-    // 128-byte line further, of a dense or LM-head call (cleared by each).
+    // x has a nonzero BF16 lo half: of a MoE call and, a 128-byte line further,
+    // of a dense or LM-head call.  Zero between calls: a kernel of the call
+    // that runs after the last reader clears it (dirty: a call ended before).
     unsigned int* lo_flag = nullptr;
-    bool lo_dirty = false;
+    bool lo_dirty = false, one_dirty = false;
     unsigned int* one_lo_flag() const { return lo_flag + 32; }
     uint16_t* xh = nullptr;      // [maxT, d] x BF16 hi (token order)
     uint16_t* xl = nullptr;      // [maxT, d] x BF16 lo
@@ -213,14 +213,19 @@ int forward_grouped(LayerState& L, const float* x, int T, float* out, hipStream_
                     const hfmoe_route_debug* dbg);
 // h += MoE(RMSNorm(h)) over the multi-token path (grouped workspace allocated).
 int forward_grouped_block(LayerState& L, float* h, int T, hipStream_t s);
+// forward_grouped of BF16 x [T, hidden] (the same bits as of its FP32 values).
+int forward_grouped_bf16(LayerState& L, const uint16_t* x, int T, float* out, hipStream_t s);
 // The three phases of forward_grouped (multi-token path, grouped workspace
 // allocated): routing (x split, router, selection, dispatch), the expert
 // gate/up and down GEMMs of the groups whose etab entries are not null (3 per
 // group, E + 1 groups, the shared expert last), and the weighted combine
 // (added to residual when given, which may be out).
 int grouped_route(LayerState& L, const float* x, int T, hipStream_t s);
-int grouped_experts(const uint16_t* const* etab, int T, hipStream_t s);
+int grouped_experts(const uint16_t* const* etab, const uint16_t* x_hi, int T, hipStream_t s);  // x_hi: gws.xh or the caller's BF16 x
 int grouped_combine(int T, const float* residual, float* out, hipStream_t s);
+// The flag of the call that begins, zero (cleared first after a call that
+// failed half-way), and dirty from here on.
+int lo_flag_begin(unsigned* flag, bool& dirty, hipStream_t s);
 int grouped_tile_rows(int T);
 int grouped_workspace_alloc();
 void grouped_workspace_free();
@@ -230,7 +235,8 @@ int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t 
 void dense_workspace_free();
 // lm_head.hip
 void lm_head_release();
-hipError_t launch_row_argmax(const float* x, int T, int n, int* out, hipStream_t s);
+// clear (may be null): one word zeroed.
+hipError_t launch_row_argmax(const float* x, int T, int n, int* out, unsigned* clear, hipStream_t s);
 hipError_t launch_matvec_bf16(const uint16_t* W, const float* x, int M, int K, float* y, hipStream_t s);
 // streamed.hip
 int streamed_forward_t1(int layer, LayerState& L, const float* x, float* out, hipStream_t s,
@@ -241,9 +247,8 @@ int streamed_forward_batch(int layer, LayerState& L, const float* x, int T, floa
                            const hfmoe_route_debug* dbg);
 void stream_pool_release();
 // misc kernels
-// clear (may be null): one word zeroed.
 hipError_t launch_rmsnorm(const float* h, const uint16_t* w, float* out, int T, int d, float eps,
-                          unsigned* clear, hipStream_t s);
+                          hipStream_t s);
 // The normalised rows as BF16 hi / lo halves; *flag (0 before) = 1 when any lo
 // half is nonzero.
 hipError_t launch_rmsnorm_split(const float* h, const uint16_t* w, uint16_t* hi, uint16_t* lo, int T, int d, float eps,
@@ -251,6 +256,9 @@ hipError_t launch_rmsnorm_split(const float* h, const uint16_t* w, uint16_t* hi,
 hipError_t launch_add_inplace(float* dst, const float* src, size_t n, hipStream_t s);
 hipError_t launch_copy_f32(const float* src, float* dst, size_t n, hipStream_t s);
 hipError_t launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStream_t s);
+// *flag (0 before) = 1 when any of x's n BF16 values is an infinity or NaN; lo
+// then holds the lo halves that the FP32 path would give (else it is untouched).
+hipError_t launch_bf16_lo(const uint16_t* x, uint16_t* lo, size_t n, unsigned* flag, hipStream_t s);
 // dst[0, n) = src[0, n) by a kernel (either may be mapped pinned host memory).
 hipError_t launch_copy_u32(const uint32_t* src, uint32_t* dst, size_t n, hipStream_t s);
 hipError_t launch_copy_u64(const uint64_t* src, uint64_t* dst, size_t n, hipStream_t s);

@@ -97,6 +97,7 @@ struct GemmArgs {
         const int* count;
         int shared_mtiles;
     } lo_tiles;
+    unsigned* clear;            // launch_fixed_gemm: one word zeroed (null: none)
 };
 
 // Groups whose b_tab entry (3g + b_which) is null are skipped.

@@ -133,7 +133,9 @@ __global__ __launch_bounds__(256) void argmax_merge_kernel(const ArgMax* __restr
 // 154880: 188 us with 256 threads and one 4-byte load each, 15 us now.
 constexpr int kArgmaxThreads = 1024;
 __global__ __launch_bounds__(kArgmaxThreads) void row_argmax_kernel(const float* __restrict__ logits, int V,
-                                                                    int* __restrict__ out) {
+                                                                    int* __restrict__ out,
+                                                                    unsigned* __restrict__ clear) {
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0u;
     constexpr int U = 4;
     __shared__ ArgMax s[kArgmaxThreads / 64];
     const int t = threadIdx.x;
@@ -181,8 +183,8 @@ static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, 
     return launch(lm_gemv_kernel<KCH, RF>, dim3(grid), dim3(kLmBlock), 0, s, W, x, V, K, logits, part);
 }
 
-hipError_t launch_row_argmax(const float* x, int T, int n, int* out, hipStream_t s) {
-    return launch(row_argmax_kernel, dim3(T), dim3(kArgmaxThreads), 0, s, x, n, out);
+hipError_t launch_row_argmax(const float* x, int T, int n, int* out, unsigned* clear, hipStream_t s) {
+    return launch(row_argmax_kernel, dim3(T), dim3(kArgmaxThreads), 0, s, x, n, out, clear);
 }
 
 static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, float* logits, ArgMax* part,
@@ -251,13 +253,12 @@ static FixedPlan lm_plan(int T, int d, int vocab, size_t split_floats, int& cb) 
 static int lm_head_forward(const float* h, int T, float* logits, int* token, hipStream_t s) {
     const Cfg& c = g.cfg;
     const LmHead& L = g.lm;
-    float* xn = g.ws.tmp;  // [T, d]
     Pending p;
-    prof_begin(p, "lm_norm", s);
     const bool gemm = T > 1 && g.gws.xh && c.d % kGemmTileK == 0;
-    HF_CHECK_LAUNCH(launch_rmsnorm(h, L.norm, xn, T, c.d, c.eps, gemm ? g.gws.one_lo_flag() : nullptr, s),
-                    "final norm");
     if (!gemm) {
+        float* xn = g.ws.tmp;  // [T, d]
+        prof_begin(p, "lm_norm", s);
+        HF_CHECK_LAUNCH(launch_rmsnorm(h, L.norm, xn, T, c.d, c.eps, s), "final norm");
         const int grid = lm_call_grid();
         for (int t = 0; t < T; ++t) {
             prof_begin(p, "lm_head_gemv", s);
@@ -273,9 +274,13 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
         }
         return HFMOE_OK;
     }
+    // The norm writes the halves the GEMM reads; the argmax, which follows it,
+    // clears their flag.
     GroupedWorkspace& gw = g.gws;
-    prof_begin(p, "split_x", s);
-    HF_CHECK_LAUNCH(launch_split_bf16(xn, gw.xh, gw.xl, (size_t)T * c.d, gw.one_lo_flag(), s), "split x");
+    const int rc = lo_flag_begin(gw.one_lo_flag(), gw.one_dirty, s);
+    if (rc) return rc;
+    prof_begin(p, "lm_norm", s);
+    HF_CHECK_LAUNCH(launch_rmsnorm_split(h, L.norm, gw.xh, gw.xl, T, c.d, c.eps, gw.one_lo_flag(), s), "final norm");
     GemmArgs a{};
     a.K = c.d;
     a.N = L.vocab;
@@ -314,8 +319,11 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     }
     if (token) {
         prof_begin(p, "lm_argmax", s);
-        HF_CHECK_LAUNCH(launch_row_argmax(logits, T, L.vocab, token, s), "argmax");
+        HF_CHECK_LAUNCH(launch_row_argmax(logits, T, L.vocab, token, gw.one_lo_flag(), s), "argmax");
+    } else {
+        HF_CHECK_LAUNCH(launch_clear_u32(gw.one_lo_flag(), 1, s), "flag clear");
     }
+    gw.one_dirty = false;
     return HFMOE_OK;
 }
 

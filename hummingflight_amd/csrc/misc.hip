@@ -11,10 +11,8 @@ namespace hf {
 constexpr int kNormThreads = 1024;
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float* __restrict__ h,
                                                                const uint16_t* __restrict__ w,
-                                                               float* __restrict__ out, int d, float eps,
-                                                               unsigned* __restrict__ clear) {
+                                                               float* __restrict__ out, int d, float eps) {
     __shared__ float red[kNormThreads / 64];
-    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0u;
     const float* x = h + (size_t)blockIdx.x * d;
     float* y = out + (size_t)blockIdx.x * d;
     const bool vec = (d & 3) == 0;
@@ -149,6 +147,48 @@ hipError_t launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, hipStre
     return launch(bf16_to_f32_kernel, dim3((unsigned)blocks), dim3(256), 0, s, src, dst, n);
 }
 
+// The lo half of a BF16 value held as FP32 is zero, but for an infinity or NaN,
+// whose difference from its own hi half is NaN.  So x goes to the multi-token
+// GEMMs as it is, and two kernels stand for the widening to FP32 and its split:
+// the first reads x (2 of the 14 bytes per value that those moved; 4096 x 6144
+// 66 -> 14 us) and flags such values, the second writes the lo halves, only
+// where there are any.
+__device__ __forceinline__ bool bf16_special(uint32_t v) { return (v & 0x7F80u) == 0x7F80u; }
+
+__global__ void bf16_specials_kernel(const uint16_t* __restrict__ x, size_t n, unsigned* __restrict__ flag) {
+    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    bool any = false;
+    auto test = [&](uint32_t w) { any |= bf16_special(w) || bf16_special(w >> 16); };
+    for (size_t i = tid; i < n / 8; i += stride) {
+        const uint4 v = reinterpret_cast<const uint4*>(x)[i];
+        test(v.x);
+        test(v.y);
+        test(v.z);
+        test(v.w);
+    }
+    if (tid < n % 8) any |= bf16_special(x[n - 1 - tid]);
+    if (__ballot(any) != 0ull && (threadIdx.x & 63) == 0) *flag = 1u;
+}
+
+__global__ void bf16_lo_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ lo, size_t n,
+                               const unsigned* __restrict__ flag) {
+    if (*flag == 0u) return;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const float v = __uint_as_float((uint32_t)x[i] << 16);
+        lo[i] = f32_to_bf16(v - __uint_as_float((uint32_t)f32_to_bf16(v) << 16));
+    }
+}
+
+hipError_t launch_bf16_lo(const uint16_t* x, uint16_t* lo, size_t n, unsigned* flag, hipStream_t s) {
+    if (reinterpret_cast<uintptr_t>(x) & 15) return hipErrorInvalidValue;
+    const size_t blocks = std::min<size_t>((n / 8 + 255) / 256 + 1, 2048);
+    hipError_t e = launch(bf16_specials_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, n, flag);
+    if (e != hipSuccess) return e;
+    return launch(bf16_lo_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, lo, n, flag);
+}
+
 __global__ void copy_u32_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, size_t n) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
@@ -172,9 +212,9 @@ hipError_t launch_copy_u64(const uint64_t* src, uint64_t* dst, size_t n, hipStre
 }
 
 hipError_t launch_rmsnorm(const float* h, const uint16_t* w, float* out, int T, int d, float eps,
-                          unsigned* clear, hipStream_t s) {
+                          hipStream_t s) {
     if (d > 8 * kNormThreads) return hipErrorInvalidValue;
-    return launch(rmsnorm_kernel, dim3(T), dim3(kNormThreads), 0, s, h, w, out, d, eps, clear);
+    return launch(rmsnorm_kernel, dim3(T), dim3(kNormThreads), 0, s, h, w, out, d, eps);
 }
 
 hipError_t launch_rmsnorm_split(const float* h, const uint16_t* w, uint16_t* hi, uint16_t* lo, int T, int d, float eps,

@@ -55,6 +55,30 @@ def test_block_of_a_batch(hf, dims, n_shared):
     r.dev.free()
 
 
+@pytest.mark.parametrize("T", [3, 24, 1024])
+def test_bf16_call_with_specials(hf, T):
+    # The BF16 call reads x itself; infinities and NaN, whose lo halves in the
+    # FP32 call are NaN, must come out as there, and a call after it as before.
+    d = SMALL["hidden"]
+    r = Run(SMALL, n_group=8, topk_group=4, seed=99, T=T)
+    bits = np.random.default_rng(T).standard_normal((T, d)).astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)
+    special = bits.copy()
+    for t, v in ((0, 0x7F800000), (T // 2, 0xFF800000), (T - 1, 0x7FC00000), (T - 1, 0xFFFF0000)):
+        special[t, 7 + t % 5] = v
+    special[0, d - 1] = 0x00010000  # a denormal
+    for x in (bits, special, bits):
+        x = x.view(np.float32)
+        xb = capi.DeviceBuffer.of((x.view(np.uint32) >> 16).astype(np.uint16))
+        out = capi.DeviceBuffer(4 * x.size)
+        capi.call("hfmoe_moe_forward_bf16", r.layer, xb.ptr, T, out.ptr, None)
+        capi.call("hfmoe_synchronize")
+        got = out.download(np.float32, x.size).reshape(x.shape)
+        assert np.array_equal(got, forward(r, x, T), equal_nan=True)
+        xb.free()
+        out.free()
+    r.dev.free()
+
+
 def test_lo_half_flag_from_call_to_call(hf):
     # An infinite router weight tells whether a BF16-valued x was multiplied
     # with lo halves: 0 * inf makes that expert's logits NaN where inf alone
@@ -74,15 +98,17 @@ def test_lo_half_flag_from_call_to_call(hf):
     xf = rng.standard_normal((T, d)).astype(np.float32)
     xb = (xf.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
     xd, xbd, out = capi.DeviceBuffer.of(xf), capi.DeviceBuffer.of(xb), capi.DeviceBuffer(4 * T * max(d, 3 * 512))
+    tok = capi.DeviceBuffer(4 * T)
     first = r.forward(xbd)["logits"]
     assert np.isinf(first[:, 3]).all() and np.isfinite(np.delete(first, 3, axis=1)).all()
     assert np.isnan(r.forward(xd)["logits"][:, 3]).any()  # the lo halves do show
     others = [lambda: block(r, xf, T), lambda: forward(r, xf, T),
               lambda: capi.call("hfmoe_dense_mlp_forward", 7, xd.ptr, T, out.ptr, None),
-              lambda: capi.call("hfmoe_lm_head", xd.ptr, T, out.ptr, None, None)]
+              lambda: capi.call("hfmoe_lm_head", xd.ptr, T, out.ptr, None, None),
+              lambda: capi.call("hfmoe_lm_head", xd.ptr, T, out.ptr, tok.ptr, None)]
     for other in others:
         other()
         assert np.array_equal(r.forward(xbd)["logits"], first)
-    for b in (table, xd, xbd, out):
+    for b in (table, xd, xbd, out, tok):
         b.free()
     r.dev.free()
