@@ -38,12 +38,17 @@ __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __res
                                                            const float* __restrict__ x, int V, int K,
                                                            float* __restrict__ logits,
                                                            ArgMax* __restrict__ part) {
-    __shared__ __attribute__((aligned(16))) float xs[KCH * 512];
+    // x in LDS, chunk ch = x[8 ch .. 8 ch + 8) split into halves xs[0][ch],
+    // xs[1][ch] so that a wavefront's 16-byte reads are consecutive: at 32-byte
+    // strides they met in half the banks, and every row pair waited for its
+    // reads (vocab 154880 x 6144 291 -> 283 us, 32000 x 2048 23.2 -> 20).
+    __shared__ float4 xs[2][KCH * 64];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int nwaves = gridDim.x * (kLmBlock / 64);
     const int gw = blockIdx.x * (kLmBlock / 64) + wave;
-    for (int i = threadIdx.x; i < KCH * 512; i += kLmBlock) xs[i] = i < K ? x[i] : 0.0f;
+    for (int i = threadIdx.x; i < KCH * 512; i += kLmBlock)  // (x may start on any 4-byte boundary)
+        reinterpret_cast<float*>(xs[(i >> 2) & 1])[(i >> 3) * 4 + (i & 3)] = i < K ? x[i] : 0.0f;
     __syncthreads();
     float best = -INFINITY;
     int best_i = INT_MAX;
@@ -64,12 +69,11 @@ __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __res
         for (int u = 0; u < RF; ++u) acc[u] = 0.0f;
         // Re-read x from LDS for every row pair: an opaque offset keeps the
         // compiler from hoisting the reads (and 96 registers) out of the loop.
-        int xo = lane * 8;
+        int xo = lane;
         asm volatile("" : "+v"(xo));
 #pragma unroll
         for (int j = 0; j < KCH; ++j) {
-            const float4 xa = *reinterpret_cast<const float4*>(xs + j * 512 + xo);
-            const float4 xb = *reinterpret_cast<const float4*>(xs + j * 512 + xo + 4);
+            const float4 xa = xs[0][j * 64 + xo], xb = xs[1][j * 64 + xo];
             const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
 #pragma unroll
             for (int u = 0; u < RF; ++u) {
