@@ -7,8 +7,7 @@
 // maximum; its OpenMP merge of per-thread winners is the same unless two
 // threads hold exactly equal maxima).
 //
-// T = 1: a persistent GEMV.  Each block stages the normalised hidden state in
-//   LDS; each wavefront streams whole vocabulary rows, two at a time, 16-byte
+// T = 1: a persistent GEMV.  Each block normalises the hidden state into LDS; each wavefront streams whole vocabulary rows, two at a time, 16-byte
 //   non-temporal loads (lane l: elements 512j + 8l .. +7; the weights are read
 //   once and kept out of the caches' way); lane 0 writes the logit and
 //   keeps the wavefront's running winner, the block merges its four, and one
@@ -33,9 +32,14 @@ __device__ __forceinline__ bool better(float va, int ia, float vb, int ib) {
 
 constexpr int kLmBlock = 256;
 
-template <int KCH, int RF>
+// NORM: x is the hidden state, and each block normalises it on the way into
+// LDS (rmsnorm_kernel's sums in its order, a thread standing for four of its:
+// the same bits): 36 KB from L2 beside the table's 3.7 MB a block, for a launch
+// less (vocab 154880 x 6144 294 -> 288 us, 32000 x 2048 27 -> 24).
+template <int KCH, int RF, bool NORM>
 __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __restrict__ W,
                                                            const float* __restrict__ x, int V, int K,
+                                                           const uint16_t* __restrict__ norm, float eps,
                                                            float* __restrict__ logits,
                                                            ArgMax* __restrict__ part) {
     // x in LDS, chunk ch = x[8 ch .. 8 ch + 8) split into halves xs[0][ch],
@@ -47,8 +51,52 @@ __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __res
     const int wave = threadIdx.x >> 6;
     const int nwaves = gridDim.x * (kLmBlock / 64);
     const int gw = blockIdx.x * (kLmBlock / 64) + wave;
-    for (int i = threadIdx.x; i < KCH * 512; i += kLmBlock)  // (x may start on any 4-byte boundary)
-        reinterpret_cast<float*>(xs[(i >> 2) & 1])[(i >> 3) * 4 + (i & 3)] = i < K ? x[i] : 0.0f;
+    if constexpr (NORM) {
+        constexpr int kOf = 1024;  // rmsnorm_kernel's threads, this block's thread t for t + 256 m
+        constexpr int M = kOf / kLmBlock, J = (KCH * 512 + 4 * kOf - 1) / (4 * kOf);
+        __shared__ float red[kOf / 64];
+        float4 v[M][J];
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const int i = 4 * ((int)threadIdx.x + m * kLmBlock + j * kOf);
+                v[m][j] = i < K ? *reinterpret_cast<const float4*>(x + i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            float sq = 0.0f;
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                sq = fmaf(v[m][j].x, v[m][j].x, sq);
+                sq = fmaf(v[m][j].y, v[m][j].y, sq);
+                sq = fmaf(v[m][j].z, v[m][j].z, sq);
+                sq = fmaf(v[m][j].w, v[m][j].w, sq);
+            }
+            sq = wave_sum(sq);
+            if (lane == 0) red[wave + m * (kLmBlock / 64)] = sq;
+        }
+        __syncthreads();
+        float tot = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kOf / 64; ++i) tot += red[i];
+        const float r = 1.0f / sqrtf(tot / (float)K + eps);
+        auto wt = [&](int i) { return norm ? __uint_as_float((uint32_t)norm[i] << 16) : 1.0f; };
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const int i = 4 * ((int)threadIdx.x + m * kLmBlock + j * kOf);
+                const float4 h = v[m][j];
+                if (i < KCH * 512)
+                    xs[(i >> 2) & 1][i >> 3] =
+                        i < K ? make_float4(h.x * r * wt(i), h.y * r * wt(i + 1), h.z * r * wt(i + 2), h.w * r * wt(i + 3))
+                              : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+    } else {
+        for (int i = threadIdx.x; i < KCH * 512; i += kLmBlock)  // (x may start on any 4-byte boundary)
+            reinterpret_cast<float*>(xs[(i >> 2) & 1])[(i >> 3) * 4 + (i & 3)] = i < K ? x[i] : 0.0f;
+    }
     __syncthreads();
     float best = -INFINITY;
     int best_i = INT_MAX;
@@ -180,24 +228,34 @@ __global__ __launch_bounds__(kArgmaxThreads) void row_argmax_kernel(const float*
     }
 }
 
+// The final norm of a logits call (part null and no norm: a plain matvec).
+struct LmNorm {
+    const uint16_t* w;  // null: ones
+    float eps;
+};
+
 template <int KCH>
-static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, float* logits, ArgMax* part,
-                               int grid, hipStream_t s) {
+static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, const LmNorm* norm, float* logits,
+                               ArgMax* part, int grid, hipStream_t s) {
     constexpr int RF = KCH <= 12 ? 2 : 1;
-    return launch(lm_gemv_kernel<KCH, RF>, dim3(grid), dim3(kLmBlock), 0, s, W, x, V, K, logits, part);
+    if (norm)
+        return launch(lm_gemv_kernel<KCH, RF, true>, dim3(grid), dim3(kLmBlock), 0, s, W, x, V, K, norm->w, norm->eps,
+                      logits, part);
+    return launch(lm_gemv_kernel<KCH, RF, false>, dim3(grid), dim3(kLmBlock), 0, s, W, x, V, K, nullptr, 0.0f, logits,
+                  part);
 }
 
 hipError_t launch_row_argmax(const float* x, int T, int n, int* out, unsigned* clear, hipStream_t s) {
     return launch(row_argmax_kernel, dim3(T), dim3(kArgmaxThreads), 0, s, x, n, out, clear);
 }
 
-static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, float* logits, ArgMax* part,
-                                 int grid, hipStream_t s) {
+static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, const LmNorm* norm, float* logits,
+                                 ArgMax* part, int grid, hipStream_t s) {
     const int kch = (K + 511) / 512;
-    if (kch <= 4) return lm_gemv_inst<4>(W, x, V, K, logits, part, grid, s);
-    if (kch <= 8) return lm_gemv_inst<8>(W, x, V, K, logits, part, grid, s);
-    if (kch <= 12) return lm_gemv_inst<12>(W, x, V, K, logits, part, grid, s);
-    if (kch <= 16) return lm_gemv_inst<16>(W, x, V, K, logits, part, grid, s);
+    if (kch <= 4) return lm_gemv_inst<4>(W, x, V, K, norm, logits, part, grid, s);
+    if (kch <= 8) return lm_gemv_inst<8>(W, x, V, K, norm, logits, part, grid, s);
+    if (kch <= 12) return lm_gemv_inst<12>(W, x, V, K, norm, logits, part, grid, s);
+    if (kch <= 16) return lm_gemv_inst<16>(W, x, V, K, norm, logits, part, grid, s);
     return hipErrorInvalidValue;
 }
 
@@ -205,7 +263,7 @@ static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K
 // ~176 registers at hidden 6144; more rows or blocks measured no faster).
 // y[M] = W[M, K] . x[K] (K a multiple of 8, at most 8192), no argmax.
 hipError_t launch_matvec_bf16(const uint16_t* W, const float* x, int M, int K, float* y, hipStream_t s) {
-    return launch_lm_gemv(W, x, M, K, y, nullptr, g.num_cus * 2, s);
+    return launch_lm_gemv(W, x, M, K, nullptr, y, nullptr, g.num_cus * 2, s);
 }
 
 static int lm_grid() { return env_int("HFMOE_LM_BLOCKS", g.num_cus * 2); }
@@ -260,13 +318,11 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     Pending p;
     const bool gemm = T > 1 && g.gws.xh && c.d % kGemmTileK == 0;
     if (!gemm) {
-        float* xn = g.ws.tmp;  // [T, d]
-        prof_begin(p, "lm_norm", s);
-        HF_CHECK_LAUNCH(launch_rmsnorm(h, L.norm, xn, T, c.d, c.eps, s), "final norm");
+        const LmNorm norm{L.norm, c.eps};
         const int grid = lm_call_grid();
         for (int t = 0; t < T; ++t) {
             prof_begin(p, "lm_head_gemv", s);
-            HF_CHECK_LAUNCH(launch_lm_gemv(L.w, xn + (size_t)t * c.d, L.vocab, c.d, logits + (size_t)t * L.vocab,
+            HF_CHECK_LAUNCH(launch_lm_gemv(L.w, h + (size_t)t * c.d, L.vocab, c.d, &norm, logits + (size_t)t * L.vocab,
                                            static_cast<ArgMax*>(L.part), grid, s),
                             "lm head gemv");
             if (token) {
