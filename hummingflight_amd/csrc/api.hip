@@ -407,11 +407,11 @@ int hfmoe_moe_forward_debug(int layer, const float* x_dev, int32_t T, float* out
         }
         return HFMOE_OK;
     }
-    if (T == 1) return forward_t1(L, x_dev, out_dev, s, dbg);
+    if (T == 1) return forward_t1(L, x_dev, nullptr, out_dev, s, dbg);
     // A debug call takes the grouped path, whose dispatch it reports.
     if (!dbg && tokenwise(T)) {
         for (int t = 0; t < T; ++t) {
-            rc = forward_t1(L, x_dev + (size_t)t * g.cfg.d, out_dev + (size_t)t * g.cfg.d, s, nullptr);
+            rc = forward_t1(L, x_dev + (size_t)t * g.cfg.d, nullptr, out_dev + (size_t)t * g.cfg.d, s, nullptr);
             if (rc) return rc;
         }
         return HFMOE_OK;
@@ -499,6 +499,18 @@ int hfmoe_mlp_block(int layer, float* h_dev, int32_t T, void* stream) {
     hipError_t e = launch_rmsnorm(h_dev, L.norm_w, xn, T, g.cfg.d, g.cfg.eps, s);
     prof_end(p, s);
     if (e != hipSuccess) return fail_hip(e, "rmsnorm launch");
+    // One token (or two, one at a time) of such a layer, or of a dense one: the
+    // last kernel adds to the residual stream (GLM-5.2 layer 117.3 -> 115.7 us,
+    // 2048 x 1024 35.4 -> 33.5; same bits).
+    if (L.dense ? T == 1 : L.location == HFMOE_EXPERTS_DEVICE && (T == 1 || tokenwise(T))) {
+        for (int t = 0; t < T; ++t) {
+            const float* x = xn + (size_t)t * g.cfg.d;
+            float* h = h_dev + (size_t)t * g.cfg.d;
+            rc = L.dense ? dense_forward_t1(L, x, h, h, s) : forward_t1(L, x, h, h, s, nullptr);
+            if (rc) return rc;
+        }
+        return HFMOE_OK;
+    }
     rc = L.dense ? hfmoe_dense_mlp_forward(layer, xn, T, mo, s) : hfmoe_moe_forward(layer, xn, T, mo, s);
     if (rc) return rc;
     prof_begin(p, "residual_add", s);

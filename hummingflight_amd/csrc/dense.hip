@@ -203,27 +203,31 @@ static int dense_fixed_forward(LayerState& L, int T, float* out, hipStream_t s) 
     return HFMOE_OK;
 }
 
+int dense_forward_t1(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s) {
+    Cfg cd = g.cfg;
+    cd.k = 0;
+    cd.I = L.dense_slice;
+    cd.n_shared = L.dense_inter / L.dense_slice;
+    float* h1 = g.dws.h1;
+    Pending p;
+    prof_begin(p, "dense_gateup", s);
+    HF_CHECK_LAUNCH(launch_gateup_t1(x, L.dev, cd, nullptr, nullptr, nullptr, h1, cd.n_shared, gu_blocks(), s),
+                    "dense gate/up launch");
+    prof_begin(p, "dense_down", s);
+    HF_CHECK_LAUNCH(launch_down_t1(h1, L.dev, cd, nullptr, nullptr, addend, out, cd.n_shared, dn_blocks(), s),
+                    "dense down launch");
+    return HFMOE_OK;
+}
+
 int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t s) {
     const Cfg& c = g.cfg;
     DenseWorkspace& w = g.dws;
     Pending p;
     const bool gemm = T > 1 && w.hh && c.d % kGemmTileK == 0 && L.dense_inter % kGemmTileK == 0;
     if (!gemm) {
-        Cfg cd = c;
-        cd.k = 0;
-        cd.I = L.dense_slice;
-        cd.n_shared = L.dense_inter / L.dense_slice;
         for (int t = 0; t < T; ++t) {
-            const float* xt = x + (size_t)t * c.d;
-            float* ot = out + (size_t)t * c.d;
-            prof_begin(p, "dense_gateup", s);
-            HF_CHECK_LAUNCH(launch_gateup_t1(xt, L.dev, cd, nullptr, nullptr, nullptr, w.h1, cd.n_shared,
-                                             gu_blocks(), s),
-                            "dense gate/up launch");
-            prof_begin(p, "dense_down", s);
-            HF_CHECK_LAUNCH(launch_down_t1(w.h1, L.dev, cd, nullptr, nullptr, nullptr, ot, cd.n_shared,
-                                           dn_blocks(), s),
-                            "dense down launch");
+            const int rc = dense_forward_t1(L, x + (size_t)t * c.d, nullptr, out + (size_t)t * c.d, s);
+            if (rc) return rc;
         }
         return HFMOE_OK;
     }

@@ -191,8 +191,7 @@ template <int ICH>
 __global__ __launch_bounds__(1024) void down_t1_kernel(const float* __restrict__ h, LayerDev L,
                                                        Cfg c, const int* __restrict__ sel,
                                                        const float* __restrict__ selw,
-                                                       const float* __restrict__ addend,
-                                                       float* __restrict__ out, int nslots,
+                                                       const float* addend, float* out, int nslots,
                                                        int rows) {
     constexpr int U = down_batch_rows(ICH);
     __shared__ float part[kMaxSlots][kDownMaxRows];

@@ -38,7 +38,8 @@ int copy_debug(const hfmoe_route_debug* dbg, int T, hipStream_t s) {
     return e == hipSuccess ? HFMOE_OK : fail_hip(e, "debug copies");
 }
 
-int forward_t1_on(LayerState& L, const float* x, float* out, hipStream_t s, const T1Buffers& b, bool profile) {
+int forward_t1_on(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s, const T1Buffers& b,
+                  bool profile) {
     const Cfg& c = g.cfg;
     const int nslots = c.k + c.n_shared;
     Pending p;
@@ -67,15 +68,16 @@ int forward_t1_on(LayerState& L, const float* x, float* out, hipStream_t s, cons
     end();
     if (e != hipSuccess) return fail_hip(e, "gate/up launch");
     begin("expert_down");
-    e = launch_down_t1(b.h, L.dev, c, b.idx, b.wts, nullptr, out, nslots, dn_blocks(), s);
+    e = launch_down_t1(b.h, L.dev, c, b.idx, b.wts, addend, out, nslots, dn_blocks(), s);
     end();
     if (e != hipSuccess) return fail_hip(e, "down launch");
     return HFMOE_OK;
 }
 
-int forward_t1(LayerState& L, const float* x, float* out, hipStream_t s, const hfmoe_route_debug* dbg) {
+int forward_t1(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s,
+               const hfmoe_route_debug* dbg) {
     const T1Buffers b{g.ws.logits, g.ws.scores, g.ws.idx, g.ws.wts, g.ws.h};
-    int rc = forward_t1_on(L, x, out, s, b, true);
+    int rc = forward_t1_on(L, x, addend, out, s, b, true);
     return rc ? rc : copy_debug(dbg, 1, s);
 }
 

@@ -198,10 +198,13 @@ struct T1Buffers {
 // forward.hip
 int gu_blocks();
 int dn_blocks();
-int forward_t1(LayerState& L, const float* x, float* out, hipStream_t s, const hfmoe_route_debug* dbg);
-// The decode launches over explicit scratch; profile = false records no timing
+int forward_t1(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s,
+               const hfmoe_route_debug* dbg);
+// The decode launches over explicit scratch; addend (may be null, or out):
+// added to the result by the last of them; profile = false records no timing
 // events (so the call creates none).
-int forward_t1_on(LayerState& L, const float* x, float* out, hipStream_t s, const T1Buffers& b, bool profile);
+int forward_t1_on(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s, const T1Buffers& b,
+                  bool profile);
 // noalloc.hip: the device address of this device's static scratch array
 // (hipGetSymbolAddress, once per device; called by hfmoe_init).
 void noalloc_setup(int device);  // never fails init: see noalloc.hip
@@ -232,6 +235,8 @@ void grouped_workspace_free();
 int gemm_blocks(int tile_rows);
 // dense.hip
 int dense_forward(LayerState& L, const float* x, int T, float* out, hipStream_t s);
+// One token over the decode GEMVs (addend: as forward_t1_on).
+int dense_forward_t1(LayerState& L, const float* x, const float* addend, float* out, hipStream_t s);
 void dense_workspace_free();
 // lm_head.hip
 void lm_head_release();

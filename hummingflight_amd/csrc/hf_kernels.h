@@ -75,7 +75,8 @@ hipError_t launch_router_select(const float* part, int ksplit, int T, const floa
 hipError_t launch_gateup_t1(const float* x, const LayerDev& L, const Cfg& c, const float2* scores,
                             int* sel_idx, float* sel_w, float* h, int nslots, int blocks,
                             hipStream_t s);
-// out[j] = sum_s weight_s * (Wd_s[j,:] . h_s) (+ addend[j] when addend is not null);
+// out[j] = sum_s weight_s * (Wd_s[j,:] . h_s) (+ addend[j] when addend is not null;
+// it may be out);
 // weight = sel_w for routed slots, 1 for shared slices.
 hipError_t launch_down_t1(const float* h, const LayerDev& L, const Cfg& c, const int* sel_idx,
                           const float* sel_w, const float* addend, float* out, int nslots,

@@ -16,6 +16,7 @@
 //   block per token finds its argmax.
 #include "hf_api_internal.h"
 #include "hf_grouped.h"
+#include "hf_norm.h"
 
 #include <climits>
 
@@ -33,8 +34,7 @@ __device__ __forceinline__ bool better(float va, int ia, float vb, int ib) {
 constexpr int kLmBlock = 256;
 
 // NORM: x is the hidden state, and each block normalises it on the way into
-// LDS (rmsnorm_kernel's sums in its order, a thread standing for four of its:
-// the same bits): 36 KB from L2 beside the table's 3.7 MB a block, for a launch
+// LDS (stage_rmsnorm: rmsnorm_kernel's bits): 36 KB from L2 beside the table's 3.7 MB a block, for a launch
 // less (vocab 154880 x 6144 294 -> 288 us, 32000 x 2048 27 -> 24).
 template <int KCH, int RF, bool NORM>
 __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __restrict__ W,
@@ -52,47 +52,9 @@ __global__ __launch_bounds__(kLmBlock) void lm_gemv_kernel(const uint16_t* __res
     const int nwaves = gridDim.x * (kLmBlock / 64);
     const int gw = blockIdx.x * (kLmBlock / 64) + wave;
     if constexpr (NORM) {
-        constexpr int kOf = 1024;  // rmsnorm_kernel's threads, this block's thread t for t + 256 m
-        constexpr int M = kOf / kLmBlock, J = (KCH * 512 + 4 * kOf - 1) / (4 * kOf);
-        __shared__ float red[kOf / 64];
-        float4 v[M][J];
-#pragma unroll
-        for (int m = 0; m < M; ++m)
-#pragma unroll
-            for (int j = 0; j < J; ++j) {
-                const int i = 4 * ((int)threadIdx.x + m * kLmBlock + j * kOf);
-                v[m][j] = i < K ? *reinterpret_cast<const float4*>(x + i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            float sq = 0.0f;
-#pragma unroll
-            for (int j = 0; j < J; ++j) {
-                sq = fmaf(v[m][j].x, v[m][j].x, sq);
-                sq = fmaf(v[m][j].y, v[m][j].y, sq);
-                sq = fmaf(v[m][j].z, v[m][j].z, sq);
-                sq = fmaf(v[m][j].w, v[m][j].w, sq);
-            }
-            sq = wave_sum(sq);
-            if (lane == 0) red[wave + m * (kLmBlock / 64)] = sq;
-        }
-        __syncthreads();
-        float tot = 0.0f;
-#pragma unroll
-        for (int i = 0; i < kOf / 64; ++i) tot += red[i];
-        const float r = 1.0f / sqrtf(tot / (float)K + eps);
-        auto wt = [&](int i) { return norm ? __uint_as_float((uint32_t)norm[i] << 16) : 1.0f; };
-#pragma unroll
-        for (int m = 0; m < M; ++m)
-#pragma unroll
-            for (int j = 0; j < J; ++j) {
-                const int i = 4 * ((int)threadIdx.x + m * kLmBlock + j * kOf);
-                const float4 h = v[m][j];
-                if (i < KCH * 512)
-                    xs[(i >> 2) & 1][i >> 3] =
-                        i < K ? make_float4(h.x * r * wt(i), h.y * r * wt(i + 1), h.z * r * wt(i + 2), h.w * r * wt(i + 3))
-                              : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
+        __shared__ float red[kNormThreads / 64];
+        static_assert(kLmBlock == kRowNormThreads, "block");
+        stage_rmsnorm<KCH>(x, norm, eps, K, xs[0], xs[1], red);
     } else {
         for (int i = threadIdx.x; i < KCH * 512; i += kLmBlock)  // (x may start on any 4-byte boundary)
             reinterpret_cast<float*>(xs[(i >> 2) & 1])[(i >> 3) * 4 + (i & 3)] = i < K ? x[i] : 0.0f;
@@ -228,14 +190,8 @@ __global__ __launch_bounds__(kArgmaxThreads) void row_argmax_kernel(const float*
     }
 }
 
-// The final norm of a logits call (part null and no norm: a plain matvec).
-struct LmNorm {
-    const uint16_t* w;  // null: ones
-    float eps;
-};
-
 template <int KCH>
-static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, const LmNorm* norm, float* logits,
+static hipError_t lm_gemv_inst(const uint16_t* W, const float* x, int V, int K, const RowNorm* norm, float* logits,
                                ArgMax* part, int grid, hipStream_t s) {
     constexpr int RF = KCH <= 12 ? 2 : 1;
     if (norm)
@@ -249,7 +205,7 @@ hipError_t launch_row_argmax(const float* x, int T, int n, int* out, unsigned* c
     return launch(row_argmax_kernel, dim3(T), dim3(kArgmaxThreads), 0, s, x, n, out, clear);
 }
 
-static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, const LmNorm* norm, float* logits,
+static hipError_t launch_lm_gemv(const uint16_t* W, const float* x, int V, int K, const RowNorm* norm, float* logits,
                                  ArgMax* part, int grid, hipStream_t s) {
     const int kch = (K + 511) / 512;
     if (kch <= 4) return lm_gemv_inst<4>(W, x, V, K, norm, logits, part, grid, s);
@@ -318,7 +274,7 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     Pending p;
     const bool gemm = T > 1 && g.gws.xh && c.d % kGemmTileK == 0;
     if (!gemm) {
-        const LmNorm norm{L.norm, c.eps};
+        const RowNorm norm{L.norm, c.eps};
         const int grid = lm_call_grid();
         for (int t = 0; t < T; ++t) {
             prof_begin(p, "lm_head_gemv", s);

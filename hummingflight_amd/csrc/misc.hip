@@ -1,6 +1,7 @@
 // misc.hip -- RMSNorm and residual add around the MoE block
 // (glm_forward.cpp:185-197 and :785-796).
 #include "hf_api_internal.h"
+#include "hf_norm.h"
 
 namespace hf {
 
@@ -8,7 +9,6 @@ namespace hf {
 // out = x*r*w (w BF16 or 1).  Each thread loads its (at most two) float4
 // chunks once and keeps them in registers for the second pass, so a token
 // costs one round trip to memory, not two.
-constexpr int kNormThreads = 1024;
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float* __restrict__ h,
                                                                const uint16_t* __restrict__ w,
                                                                float* __restrict__ out, int d, float eps) {

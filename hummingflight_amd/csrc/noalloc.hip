@@ -111,7 +111,7 @@ int hfmoe_moe_forward_noalloc(int layer, const float* x_dev, int32_t T, float* o
     const T1Buffers b{reinterpret_cast<float*>(base + off[0]), reinterpret_cast<float2*>(base + off[1]),
                       reinterpret_cast<int*>(base + off[2]), reinterpret_cast<float*>(base + off[3]),
                       reinterpret_cast<float*>(base + off[4])};
-    return forward_t1_on(L, x_dev, out_dev, pick_stream(stream), b, false);
+    return forward_t1_on(L, x_dev, nullptr, out_dev, pick_stream(stream), b, false);
 }
 
 }  // extern "C"

@@ -45,7 +45,7 @@ def test_block_of_a_batch(hf, dims, n_shared):
     r = Run(dims, n_group=4, topk_group=2, seed=97, T=most, n_shared=n_shared, with_norm=True)
     w = O.bf16_to_f32(r.dev.norm.download(np.uint16, d))
     rng = np.random.default_rng(97)
-    for T in (2, 3, 5, 17, 260):
+    for T in (1, 2, 3, 5, 17, 260):
         h = (3.0 * rng.standard_normal((T, d))).astype(np.float32)
         xn = (h * (1.0 / np.sqrt((h * h).mean(1, dtype=np.float32, keepdims=True) + np.float32(1e-5)))).astype(
             np.float32) * w
