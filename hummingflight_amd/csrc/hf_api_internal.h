@@ -56,7 +56,7 @@ struct GroupedWorkspace {
     uint16_t* xl = nullptr;      // [maxT, d] x BF16 lo
     uint16_t* hh = nullptr;      // [rows, I] h hi (sorted rows)
     uint16_t* hl = nullptr;      // [rows, I] h lo
-    float* y = nullptr;          // [rows, d] expert outputs at pair slots, shared rows after
+    float* y = nullptr;          // [rows, d] expert outputs at pair slots, shared rows after (LM head: K-split partials)
     float* part = nullptr;       // [ksplit, maxT, E] router split-K partials
     int max_tiles = 0;
 };
@@ -83,9 +83,6 @@ struct LmHead {
     int vocab = 0;
     void* part = nullptr;            // per-block winners of the T = 1 GEMV
     int part_n = 0;                  // their number: the most workgroups that GEMV takes
-    float* split = nullptr;          // K-split partials of the multi-token GEMM, or null
-    size_t split_floats = 0;
-    float* split_own = nullptr;      // the allocation behind them, if they have one
 };
 
 // Buffers of the dense-MLP layers (sized for the largest registered inter).

@@ -229,7 +229,6 @@ static int lm_call_grid() { return std::max(1, std::min(lm_grid(), g.lm.part_n))
 
 void lm_head_release() {
     if (g.lm.part) hipFree(g.lm.part);
-    if (g.lm.split_own) hipFree(g.lm.split_own);
     g.lm = LmHead{};
 }
 
@@ -249,22 +248,24 @@ void lm_head_release() {
 // 335-350, 24 377 against 335, 64 490 against 361, 128 690 against 430; T =
 // 300 1673 on 256-row tiles against 1114).
 constexpr int kLmFixedTokens = 17;
-constexpr size_t kLmSplitFloats = (size_t)64 << 20;  // K-split partials: as many are plenty
-static FixedPlan lm_plan(int T, int d, int vocab, size_t split_floats, int& cb) {
+static FixedPlan lm_plan(int T, int d, int vocab, int& cb) {
     FixedPlan best;
     cb = 0;
     if (T < kLmFixedTokens || !fixed_worth(T, (size_t)vocab * d)) return best;
+    // K-split partials go to the MoE path's y rows (the split sum adds four
+    // logits at a time).
+    const size_t one = (size_t)T * vocab, y_floats = (size_t)g.max_tokens * (g.cfg.k + g.cfg.n_shared) * g.cfg.d;
+    const int splits = one % 4 ? 1 : (int)std::max((size_t)1, std::min((size_t)kFixedMaxSplits, y_floats / one));
     for (int c = 4; c <= 5; ++c) {
         if (vocab < fixed_tile_cols(c, false) || (c == 5 && T > fixed_tile_rows(5))) continue;
-        // (the split sum adds four logits at a time)
-        const size_t one = (size_t)T * vocab;
-        const int splits = one % 4 ? 1 : (int)std::max((size_t)1, std::min((size_t)kFixedMaxSplits, split_floats / one));
         const FixedPlan pl = plan_fixed_gemm(T, vocab, false, c, d / kGemmTileK, splits, g.num_cus);
         if (!cb || pl.us < best.us) {
             best = pl;
             cb = c;
         }
     }
+    // A short table without room for the splits that fill the chip.
+    if (T <= kGemmTileRows && 2 * best.m_tiles * best.n_tiles * best.ksplit < g.num_cus) cb = 0;
     return best;
 }
 
@@ -309,18 +310,18 @@ static int lm_head_forward(const float* h, int T, float* logits, int* token, hip
     a.out_f32 = logits;
     a.ksplit = 1;
     int cb = 0;
-    const FixedPlan pl = lm_plan(T, c.d, L.vocab, L.split_floats, cb);
+    const FixedPlan pl = lm_plan(T, c.d, L.vocab, cb);
     if (cb) {
         a.tile_rows = pl.tile_rows;
         a.m_tiles = pl.m_tiles;
         a.n_tiles = pl.n_tiles;
         a.ksplit = pl.ksplit;
-        if (pl.ksplit > 1) a.out_f32 = L.split;
+        if (pl.ksplit > 1) a.out_f32 = gw.y;
         prof_begin(p, "lm_head_gemm", s);
         HF_CHECK_LAUNCH(launch_fixed_gemm(EPI_PARTIAL, false, cb, a, gemm_blocks(kPrefillTileRows), s), "lm head gemm");
         if (pl.ksplit > 1) {
             prof_begin(p, "lm_head_sum", s);
-            HF_CHECK_LAUNCH(launch_sum_splits(L.split, pl.ksplit, (size_t)T * L.vocab, logits, s), "lm head split sum");
+            HF_CHECK_LAUNCH(launch_sum_splits(gw.y, pl.ksplit, (size_t)T * L.vocab, logits, s), "lm head split sum");
         }
     } else {
         // Past one 128-row M tile (a table shorter than one 512-row tile), the
@@ -360,29 +361,6 @@ int hfmoe_register_lm_head(const uint16_t* lm_head_dev, const uint16_t* final_no
     const int part_n = std::max(1, lm_grid());
     hipError_t e = hipMalloc(&g.lm.part, sizeof(ArgMax) * (size_t)part_n);
     if (e != hipSuccess) return fail_hip(e, "lm head workspace");
-    // K-split partials of the multi-token GEMM: the MoE path's y rows where
-    // they are plenty, else a buffer for what the plans take.
-    const size_t y_floats = g.gws.xh ? (size_t)g.max_tokens * (g.cfg.k + g.cfg.n_shared) * g.cfg.d : 0;
-    if (y_floats >= kLmSplitFloats) {
-        g.lm.split = g.gws.y;
-        g.lm.split_floats = y_floats;
-    } else if (g.gws.xh) {
-        size_t floats = 0;
-        for (int t = 32; t <= std::min((g.max_tokens + 15) / 16 * 16, 512); t += 16) {
-            int cb = 0;
-            const FixedPlan pl = lm_plan(t, g.cfg.d, vocab, kLmSplitFloats, cb);
-            if (pl.ksplit > 1) floats = std::max(floats, (size_t)pl.ksplit * t * vocab);
-        }
-        if (floats) {
-            e = hipMalloc(&g.lm.split_own, sizeof(float) * floats);
-            if (e != hipSuccess) {
-                lm_head_release();
-                return fail_hip(e, "lm head workspace");
-            }
-            g.lm.split = g.lm.split_own;
-            g.lm.split_floats = floats;
-        }
-    }
     g.lm.part_n = part_n;
     g.lm.w = lm_head_dev;
     g.lm.norm = final_norm_dev;
