@@ -128,7 +128,10 @@ int grouped_workspace_alloc() {
                         hipGetErrorString(e));
         }
     }
-    hipError_t e = hipMemset(w.lo_flag, 0, 256);  // zero between MoE calls
+    // Zero between MoE calls; waited for, as a caller's stream need not wait
+    // for the null stream's work.
+    hipError_t e = hipMemset(w.lo_flag, 0, 256);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return fail_hip(e, "hipMemset(flag)");
     return HFMOE_OK;
 }
